@@ -47,17 +47,16 @@ template <typename V, int DIR> struct Butterfly<V, 3, DIR> {
     using T = decltype(v[0].x);
     const T h = (T)0.86602540378443864676;  // sqrt(3)/2
     V t = cadd(v[1], v[2]);
-    V d = csub(v[1], v[2]);
+    V d = mul_si<DIR>(csub(v[1], v[2]));
     V a0 = v[0];
     V m;  // a0 - t/2
     m.x = a0.x - (T)0.5 * t.x;
     m.y = a0.y - (T)0.5 * t.y;
-    V u = mul_si<DIR>(d);  // s*i*(a1-a2)
-    u.x *= h;
-    u.y *= h;
     v[0] = cadd(a0, t);
-    v[1] = cadd(m, u);
-    v[2] = csub(m, u);
+    v[1].x = m.x + h * d.x;
+    v[1].y = m.y + h * d.y;
+    v[2].x = m.x - h * d.x;
+    v[2].y = m.y - h * d.y;
   }
 };
 
