@@ -155,12 +155,13 @@ static void build_sphere(amdk_ctx* c, const int* mill, int ncaller, Sphere& S) {
   // full rows -> slots sorted by (m3, m2)
   struct FR { int m3, m2, row, mirror; };
   std::vector<FR> fr;
-  S.R = 0;
+  S.R = S.R2 = 0;
   for (int r = 0; r < S.nrow; ++r) {
     const RowInfo& ri = S.h_rows[r];
     fr.push_back({ri.m3, ri.m2, r, 0});
     if (!(ri.m2 == 0 && ri.m3 == 0)) fr.push_back({-ri.m3, -ri.m2, r, 1});
     S.R = std::max(S.R, std::abs(ri.m3));
+    S.R2 = std::max(S.R2, std::abs(ri.m2));
   }
   std::sort(fr.begin(), fr.end(), [](const FR& x, const FR& y) { return std::make_pair(x.m3, x.m2) < std::make_pair(y.m3, y.m2); });
   S.nslot = (int)fr.size();
@@ -311,13 +312,19 @@ template <typename T, int TM> struct RegTiles {
   static constexpr int PG = sizeof(T) == 4 ? 4 : 2;
 };
 
+// Whether every |m| of a sphere's axis is at most a quarter of the grid (QW of
+// the z and y passes).
+static bool quarter_z(const Sphere& S, int n3) { return 4 * S.R <= n3; }
+static bool quarter_y(const Sphere& S, int n2) { return 4 * S.R2 <= n2; }
+
 template <typename T, int A, int B>
 static void reg_z_vpsi(amdk_ctx* c, const Sphere& S, int np) {
   using V = typename cplx_of<T>::type;
   constexpr int N = A * B, TM = MaxAB<A, B>::v, TX = RegTiles<T, TM>::ZTX, PG = RegTiles<T, TM>::PG;
   const size_t lds = (size_t)(N + N * TX) * sizeof(V);
   const int ncb = (c->n1 * c->n2 + TX - 1) / TX, ngrp = (np + PG - 1) / PG, per = (ncb * ngrp + 7) / 8;
-  k_z_vpsi_r<T, A, B, TX><<<8 * per, TX * TM, lds, c->stream>>>(geom_of(c, S), (V*)c->W2, (const T*)c->vr, np, PG,
+  auto kern = quarter_z(S, N) ? k_z_vpsi_r<T, A, B, TX, true> : k_z_vpsi_r<T, A, B, TX, false>;
+  kern<<<8 * per, TX * TM, lds, c->stream>>>(geom_of(c, S), (V*)c->W2, (const T*)c->vr, np, PG,
                                                                (const V*)(sizeof(T) == 4 ? c->tw_f[2] : c->tw_d[2]),
                                                                ngrp, per);
 }
@@ -328,7 +335,8 @@ static void reg_z_rho(amdk_ctx* c, const Sphere& S, int np, double* rho, int acc
   constexpr int N = A * B, TM = MaxAB<A, B>::v, TX = RegTiles<T, TM>::ZTX;
   const size_t lds = (size_t)(N + N * TX) * sizeof(V);
   const int ncb = (c->n1 * c->n2 + TX - 1) / TX, per = (ncb * groups + 7) / 8;
-  k_z_rho_r<T, A, B, TX><<<8 * per, TX * TM, lds, c->stream>>>(geom_of(c, S), (const V*)c->W2, rho, np, wpair, accumulate,
+  auto kern = quarter_z(S, N) ? k_z_rho_r<T, A, B, TX, true> : k_z_rho_r<T, A, B, TX, false>;
+  kern<<<8 * per, TX * TM, lds, c->stream>>>(geom_of(c, S), (const V*)c->W2, rho, np, wpair, accumulate,
                                                               (const V*)(sizeof(T) == 4 ? c->tw_f[2] : c->tw_d[2]),
                                                               part_stride, groups, per);
 }
@@ -339,10 +347,14 @@ static void reg_cols(amdk_ctx* c, const Sphere& S, int np, bool inverse) {
   const size_t lds = (size_t)(N + N * TX) * sizeof(V);
   dim3 grid((c->n1 + TX - 1) / TX, S.nplane, np);
   const V* tw = (const V*)(sizeof(T) == 4 ? c->tw_f[1] : c->tw_d[1]);
-  if (inverse)
-    k_cols_inv_r<T, A, B, TX><<<grid, TX * TM, lds, c->stream>>>(geom_of(c, S), (const V*)c->W1, (V*)c->W2, tw);
-  else
-    k_cols_fwd_r<T, A, B, TX><<<grid, TX * TM, lds, c->stream>>>(geom_of(c, S), (const V*)c->W2, (V*)c->W1, tw);
+  const bool q = quarter_y(S, N);
+  if (inverse) {
+    auto kern = q ? k_cols_inv_r<T, A, B, TX, true> : k_cols_inv_r<T, A, B, TX, false>;
+    kern<<<grid, TX * TM, lds, c->stream>>>(geom_of(c, S), (const V*)c->W1, (V*)c->W2, tw);
+  } else {
+    auto kern = q ? k_cols_fwd_r<T, A, B, TX, true> : k_cols_fwd_r<T, A, B, TX, false>;
+    kern<<<grid, TX * TM, lds, c->stream>>>(geom_of(c, S), (const V*)c->W2, (V*)c->W1, tw);
+  }
 }
 template <typename T, int A, int B>
 static void reg_rows_inv(amdk_ctx* c, const Sphere& S, const void* C, int ldc, int nb, int pair0, int np) {

@@ -46,6 +46,7 @@ struct Sphere {
   int nrow = 0;       // half rows
   int nslot = 0;      // full rows (direct + mirrored)
   int R = 0;          // max |m3|; planes are m3 = -R..R
+  int R2 = 0;         // max |m2|
   int nplane = 0;     // 2R+1
   RowInfo* rows = nullptr;      // device [nrow]
   int* slot_m2 = nullptr;       // device [nslot]

@@ -127,17 +127,58 @@ __device__ __forceinline__ void col_fft(V* r, int t, V* lds, int stride, int cof
 
 __device__ __forceinline__ int signed_freq(int p, int n) { return 2 * p <= n ? p : p - n; }
 
-// Element offset, in a pencil of planes or rows spaced `ps` apart, of the
-// frequency signed_freq(t + A k, N) relative to the first stored one (-lo),
-// or -1 when the frequency lies outside [lo, hi].  Written so that the
-// per-element work is adds and compares on `base` = (t - lo) * ps, hoisted by
-// the caller, instead of 64-bit index products.
+// One pencil of planes (or of a plane's rows) as a bounded buffer: elements
+// of V at unsigned byte offsets below `bytes` of the wave-uniform base.  The
+// hardware returns 0 for a load past the end and drops a store there, so the
+// sphere's edges need no compare, branch or mask: frequencies above the last
+// stored one lie past the end, those below the first at negative offsets,
+// which are past it as unsigned numbers, and a thread without a column starts
+// at DEAD_OFF.  Buffers are below 2^31 - 2^27 bytes (grids up to 192^3: 113 MB).
+// The masked accesses this replaced took a third of z_vpsi's vector
+// instructions (891 -> 614 with the quarter window below) and its loads were
+// parted by branches: z_vpsi 0.168 -> 0.132 ms at 32 H2O (FP64 0.277 ->
+// 0.214), 0.80 -> 0.60 ms at 64 H2O; z_rho 0.094 -> 0.090 and 0.43 -> 0.39 ms.
+// The y passes, bound by memory, gained nothing by it (0.072 -> 0.074 ms).
+typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+constexpr unsigned DEAD_OFF = 0x80000000u;
+
+template <typename V> struct PencilBuf {
+  __amdgpu_buffer_rsrc_t rs;
+  __device__ __forceinline__ PencilBuf(const V* p, unsigned bytes)
+      : rs(__builtin_amdgcn_make_buffer_rsrc(const_cast<V*>(p), 0, bytes, 0x00027000)) {}
+  __device__ __forceinline__ V load(unsigned off) const {
+    if constexpr (sizeof(V) == 8) return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0));
+    else return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+  }
+  __device__ __forceinline__ void store(unsigned off, V v) const {
+    if constexpr (sizeof(V) == 8) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2v, v), rs, off, 0, 0);
+    else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4v, v), rs, off, 0, 0);
+  }
+};
+
+// Position t + A k of a length-N transform relative to position t, in steps
+// of the pencil, with the upper half wrapped to negative frequencies.  Which
+// half an element falls in is known at compile time except where the middle
+// lies inside the run of A positions; N/2 itself is never stored, so either
+// side does.
 template <int A, int N>
-__device__ __forceinline__ int pencil_off(int t, int k, int lo, int hi, int base, int ps) {
-  const int z = t + A * k;
-  const bool wrap = 2 * z > N;
-  const int f = wrap ? z - N : z;
-  return (f >= lo && f <= hi) ? base + (A * k) * ps - (wrap ? N * ps : 0) : -1;
+__device__ __forceinline__ int pencil_step(int t, int k) {
+  if (2 * A * k >= N) return A * k - N;
+  if (2 * (A * k + A - 1) <= N) return A * k;
+  return 2 * (t + A * k) > N ? A * k - N : A * k;
+}
+
+// Whether a run of positions t + A k, t < A, can hold a stored frequency.  The
+// wavefunction sphere reaches at most a quarter of the grid (|m| <= N/4: the
+// grid holds the density, whose sphere is twice as wide), and QW says that it
+// does, so that the middle runs are left out at compile time: they are zeros
+// to the transform and cost no access.  A run-time test per run, which would
+// also skip what a particular plane lacks, measured slower (its branches part
+// the loads; z_vpsi at 32 H2O 0.167 instead of 0.142 ms).
+template <bool QW, int A, int N>
+constexpr bool pencil_run(int k) {
+  return !QW || 4 * A * k <= N || 4 * (N - A * k - A + 1) <= N;
 }
 
 // Block order of the z passes: MI355X hands consecutive workgroups
@@ -156,7 +197,7 @@ __device__ __forceinline__ bool z_block_of(int ngrp, int per, int ncb, int& cb, 
 
 // ---------------------------------------------------------------------------
 // z pass of H|psi>: planes |m3| <= R -> z-FFT exp(+i) -> * v(r) -> z-FFT exp(-i)
-template <typename T, int A, int B, int TX>
+template <typename T, int A, int B, int TX, bool QW>
 __global__ void __launch_bounds__(TX * (A > B ? A : B))
     k_z_vpsi_r(PassGeom g, typename cplx_of<T>::type* __restrict__ W2, const T* __restrict__ vr, int npairs,
                int PG, const typename cplx_of<T>::type* __restrict__ twg, int ngrp, int per) {
@@ -186,19 +227,15 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
   }
   __syncthreads();
   const int pg0 = grp * PG, pg1 = min(npairs, pg0 + PG);
-  const int ps = n2 * g.p1, base = (t + g.R) * ps;  // plane stride; plane kz sits at kz + R
-  const bool act = t < A && live;
+  const int ps = n2 * g.p1, psb = ps * sizeof(V);  // plane stride; plane kz sits at kz + R
+  const unsigned base = t < A && live ? (t + g.R) * psb + (y * g.p1 + x) * (unsigned)sizeof(V) : DEAD_OFF;
   for (int pl = pg0; pl < pg1; ++pl) {
-    V* col = W2 + (size_t)pl * g.nplane * ps + (size_t)y * g.p1 + x;
+    const PencilBuf<V> buf(W2 + (size_t)pl * g.nplane * ps, g.nplane * psb);
     V r[TM];
 #pragma unroll
-    for (int k = 0; k < TM; ++k) { r[k].x = 0; r[k].y = 0; }
-    if (act) {
-#pragma unroll
-      for (int k2 = 0; k2 < B; ++k2) {
-        const int o = pencil_off<A, N>(t, k2, -g.R, g.R, base, ps);
-        if (o >= 0) r[k2] = col[o];
-      }
+    for (int k2 = 0; k2 < B; ++k2) {
+      if (pencil_run<QW, A, N>(k2)) r[k2] = buf.load(base + pencil_step<A, N>(t, k2) * psb);
+      else r[k2].x = r[k2].y = 0;
     }
     col_fft<V, A, B, +1>(r, t, lds, TX, c, tw);
     if (t < B) {
@@ -209,13 +246,9 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
       }
     }
     col_fft<V, B, A, -1>(r, t, lds, TX, c, tw);
-    if (act) {
 #pragma unroll
-      for (int j1 = 0; j1 < B; ++j1) {
-        const int o = pencil_off<A, N>(t, j1, -g.R, g.R, base, ps);
-        if (o >= 0) col[o] = r[j1];
-      }
-    }
+    for (int j1 = 0; j1 < B; ++j1)
+      if (pencil_run<QW, A, N>(j1)) buf.store(base + pencil_step<A, N>(t, j1) * psb, r[j1]);
   }
 }
 
@@ -223,7 +256,7 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
 // in FP64 registers (each thread owns fixed z), ordered over pairs.  The
 // pairs are split into gridDim.z consecutive groups; group k accumulates
 // into the grid rho + k * part_stride (summed afterwards in a fixed order).
-template <typename T, int A, int B, int TX>
+template <typename T, int A, int B, int TX, bool QW>
 __global__ void __launch_bounds__(TX * (A > B ? A : B))
     k_z_rho_r(PassGeom g, const typename cplx_of<T>::type* __restrict__ W2, double* __restrict__ rho, int npairs,
               const double* __restrict__ wpair, int accumulate, const typename cplx_of<T>::type* __restrict__ twg,
@@ -249,15 +282,14 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
   // registers while this one is transformed (wider forms would lose occupancy)
   constexpr bool PF = sizeof(T) == 4 && TM <= 10;
   V rn[B];
-  const int ps = n2 * g.p1, base = (t + g.R) * ps;  // plane stride; plane kz sits at kz + R
-  const bool act = t < A && live;
+  const int ps = n2 * g.p1, psb = ps * sizeof(V);  // plane stride; plane kz sits at kz + R
+  const unsigned base = t < A && live ? (t + g.R) * psb + (y * g.p1 + x) * (unsigned)sizeof(V) : DEAD_OFF;
   auto load_pair = [&](int pl, V* dst) {
-    const V* col = W2 + (size_t)pl * g.nplane * ps + (size_t)y * g.p1 + x;
+    const PencilBuf<V> buf(W2 + (size_t)pl * g.nplane * ps, g.nplane * psb);
 #pragma unroll
     for (int k2 = 0; k2 < B; ++k2) {
-      const int o = act ? pencil_off<A, N>(t, k2, -g.R, g.R, base, ps) : -1;
-      if (o >= 0) dst[k2] = col[o];
-      else { dst[k2].x = 0; dst[k2].y = 0; }
+      if (pencil_run<QW, A, N>(k2)) dst[k2] = buf.load(base + pencil_step<A, N>(t, k2) * psb);
+      else dst[k2].x = dst[k2].y = 0;
     }
   };
   const int ppg = (npairs + ngrp - 1) / ngrp;
@@ -266,8 +298,6 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
   if (PF && pa < pb) load_pair(pa, rn);
   for (int pl = pa; pl < pb; ++pl) {
     V r[TM];
-#pragma unroll
-    for (int k = 0; k < TM; ++k) { r[k].x = 0; r[k].y = 0; }
     if constexpr (PF) {
 #pragma unroll
       for (int k2 = 0; k2 < B; ++k2) r[k2] = rn[k2];
@@ -294,7 +324,7 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
 }
 
 // y pass inverse: rows of plane m3 (consecutive m2 from m2_lo) -> y-FFT exp(+i)
-template <typename T, int A, int B, int TX>
+template <typename T, int A, int B, int TX, bool QW>
 __global__ void __launch_bounds__(TX * (A > B ? A : B))
     k_cols_inv_r(PassGeom g, const typename cplx_of<T>::type* __restrict__ W1, typename cplx_of<T>::type* __restrict__ W2,
                  const typename cplx_of<T>::type* __restrict__ twg) {
@@ -310,19 +340,16 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
   const bool live = x < n1;
   for (int i = threadIdx.x; i < N; i += blockDim.x) tw[i] = twg[i];
   const int s0 = g.plane_off[plane], s1 = g.plane_off[plane + 1];
-  const int lo = s1 > s0 ? g.slot_m2[s0] : 0, hi = lo + (s1 - s0) - 1;
+  const int lo = s1 > s0 ? g.slot_m2[s0] : 0;
   __syncthreads();
   V r[TM];
+  const int psb = g.p1 * sizeof(V);
+  const PencilBuf<V> rows(W1 + ((size_t)pl * g.nslot + s0) * g.p1, (s1 - s0) * psb);  // rows m2 = lo, lo + 1, ...
+  const unsigned base = t < A && live ? (t - lo) * psb + x * (unsigned)sizeof(V) : DEAD_OFF;
 #pragma unroll
-  for (int k = 0; k < TM; ++k) { r[k].x = 0; r[k].y = 0; }
-  if (t < A && live) {
-    const V* rows = W1 + ((size_t)pl * g.nslot + s0) * g.p1 + x;  // row of m2 = lo
-    const int base = (t - lo) * g.p1;
-#pragma unroll
-    for (int k2 = 0; k2 < B; ++k2) {
-      const int o = pencil_off<A, N>(t, k2, lo, hi, base, g.p1);
-      if (o >= 0) r[k2] = rows[o];
-    }
+  for (int k2 = 0; k2 < B; ++k2) {
+    if (pencil_run<QW, A, N>(k2)) r[k2] = rows.load(base + pencil_step<A, N>(t, k2) * psb);
+    else r[k2].x = r[k2].y = 0;
   }
   col_fft<V, A, B, +1>(r, t, lds, TX, c, tw);
   if (t < B && live) {
@@ -333,7 +360,7 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
 }
 
 // y pass forward: full plane column -> y-FFT exp(-i) -> rows inside the sphere
-template <typename T, int A, int B, int TX>
+template <typename T, int A, int B, int TX, bool QW>
 __global__ void __launch_bounds__(TX * (A > B ? A : B))
     k_cols_fwd_r(PassGeom g, const typename cplx_of<T>::type* __restrict__ W2, typename cplx_of<T>::type* __restrict__ W1,
                  const typename cplx_of<T>::type* __restrict__ twg) {
@@ -349,7 +376,7 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
   const bool live = x < n1;
   for (int i = threadIdx.x; i < N; i += blockDim.x) tw[i] = twg[i];
   const int s0 = g.plane_off[plane], s1 = g.plane_off[plane + 1];
-  const int lo = s1 > s0 ? g.slot_m2[s0] : 0, hi = lo + (s1 - s0) - 1;
+  const int lo = s1 > s0 ? g.slot_m2[s0] : 0;
   __syncthreads();
   V r[TM];
 #pragma unroll
@@ -360,15 +387,12 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
     for (int k2 = 0; k2 < B; ++k2) r[k2] = in[(A * k2) * g.p1];
   }
   col_fft<V, A, B, -1>(r, t, lds, TX, c, tw);
-  if (t < B && live) {
-    V* rows = W1 + ((size_t)pl * g.nslot + s0) * g.p1 + x;  // row of m2 = lo
-    const int base = (t - lo) * g.p1;
+  const int psb = g.p1 * sizeof(V);
+  const PencilBuf<V> rows(W1 + ((size_t)pl * g.nslot + s0) * g.p1, (s1 - s0) * psb);  // rows m2 = lo, lo + 1, ...
+  const unsigned base = t < B && live ? (t - lo) * psb + x * (unsigned)sizeof(V) : DEAD_OFF;
 #pragma unroll
-    for (int j1 = 0; j1 < A; ++j1) {
-      const int o = pencil_off<B, N>(t, j1, lo, hi, base, g.p1);
-      if (o >= 0) rows[o] = r[j1];
-    }
-  }
+  for (int j1 = 0; j1 < A; ++j1)
+    if (pencil_run<QW, B, N>(j1)) rows.store(base + pencil_step<B, N>(t, j1) * psb, r[j1]);
 }
 
 // x pass inverse: gather half rows of two bands, pack psi1 + i psi2 on the
