@@ -1,4 +1,4 @@
-// Register-resident pencil FFT passes for lengths N = A*B (A, B <= 16).
+// Register-resident pencil FFT passes for lengths N = A*B (A, B <= 18).
 //
 // One transform of length N is spread over max(A, B) threads: each thread
 // first does a length-B DFT in registers over elements t + A*k2, multiplies
@@ -26,6 +26,7 @@ template <> struct Split<10> { static constexpr int P = 2, Q = 5; };
 template <> struct Split<12> { static constexpr int P = 3, Q = 4; };
 template <> struct Split<15> { static constexpr int P = 3, Q = 5; };
 template <> struct Split<16> { static constexpr int P = 4, Q = 4; };
+template <> struct Split<18> { static constexpr int P = 2, Q = 9; };
 
 constexpr int gcd_of(int a, int b) { return b == 0 ? a : gcd_of(b, a % b); }
 
@@ -45,7 +46,7 @@ __device__ __forceinline__ V mul_root(V a, int m) {
 }
 
 // In-register DFT of x[0..L): X_k = sum_j x_j exp(DIR 2 pi i jk / L).
-// L = P Q with coprime P, Q (6, 10, 12, 15) takes the prime-factor map
+// L = P Q with coprime P, Q (6, 10, 12, 15, 18) takes the prime-factor map
 // j = Q a + P b (mod L), k -> (k mod P, k mod Q), which needs no twiddle
 // between the P- and the Q-point DFTs; 8, 9 and 16 keep the twiddled split.
 // Against the twiddled split at every length the z pass of H|psi> issues 10 %

@@ -1,0 +1,59 @@
+"""H|psi> and the density at every transform length of the register passes
+that the other tests leave out (three at a time, one per axis), and with a
+wavefunction sphere wider than a quarter of the grid, where no frequency run
+may be left out of the z and y passes."""
+import numpy as np
+import pytest
+
+from amdkiit_amd.context import KSContext
+from amdkiit_amd.pwgrid import Cell, PWSetup
+from oracle import pw_oracle as O
+from tests.common import random_bands, smooth_potential
+
+pytestmark = pytest.mark.gpu
+
+GRIDS = [(32, 40, 50), (54, 64, 80), (90, 96, 120), (128, 150, 20), (24, 160, 162), (192, 36, 30), (30, 20, 192),
+         (162, 128, 32), (50, 90, 64), (40, 54, 96), (64, 32, 90), (80, 48, 54), (96, 50, 40), (120, 80, 48), (150, 24, 60)]
+
+
+def rel(a, b):
+    return np.abs(a - b).max() / np.abs(b).max()
+
+
+def sphere_to_the_edge(n):
+    """A box whose density sphere reaches the largest |m| < n/2 of each axis."""
+    return PWSetup(Cell(np.diag([0.25 * k for k in n])), 0.24 * (2 * np.pi / 0.5) ** 2, n=n)
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("mixed", 2e-6)])
+@pytest.mark.parametrize("n", GRIDS, ids=lambda n: "x".join(map(str, n)))
+def test_lengths(n, prec, tol):
+    pw = sphere_to_the_edge(n)
+    nb = 3
+    print(f"case=lengths n={n} ngpw={pw.ngpw} R={np.abs(pw.mill_pw).max(0)} prec={prec}", flush=True)
+    c = random_bands(pw, nb, seed=3)
+    occ = np.array([2.0, 1.0, 2.0])
+    v = smooth_potential(pw)
+    ctx = KSContext(pw, nb, prec)
+    ctx.set_vks(v)
+    assert rel(ctx.vpsi(c, occ), O.vpsi(c, occ, v, pw.mill_pw, pw.n, pw.cell.g)) < tol
+    assert rel(ctx.eval_density(c, occ), O.eval_density(c, occ, pw.mill_pw, pw.n, pw.cell.omega)) < tol
+    ctx.close()
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("mixed", 2e-6)])
+@pytest.mark.parametrize("n", [(30, 32, 36), (40, 50, 54), (64, 60, 72), (100, 24, 80)], ids=lambda n: "x".join(map(str, n)))
+def test_sphere_wider_than_a_quarter_of_the_grid(n, prec, tol):
+    pw = sphere_to_the_edge(n)
+    pw.mill_pw, pw.ngpw = pw.mill_rho, pw.ngrho  # |m| up to n/2 - 1
+    assert (4 * np.abs(pw.mill_pw).max(0) > np.array(n)).all()
+    nb = 10  # density in pair groups too
+    print(f"case=wide n={n} ngpw={pw.ngpw} R={np.abs(pw.mill_pw).max(0)} prec={prec}", flush=True)
+    c = random_bands(pw, nb, seed=4)
+    occ = np.full(nb, 2.0)
+    v = smooth_potential(pw)
+    ctx = KSContext(pw, nb, prec)
+    ctx.set_vks(v)
+    assert rel(ctx.vpsi(c, occ), O.vpsi(c, occ, v, pw.mill_pw, pw.n, pw.cell.g)) < tol
+    assert rel(ctx.eval_density(c, occ), O.eval_density(c, occ, pw.mill_pw, pw.n, pw.cell.omega)) < tol
+    ctx.close()
