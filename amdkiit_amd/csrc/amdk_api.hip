@@ -10,7 +10,7 @@
 #include <tuple>
 
 #include "amdk_ctx.h"
-#include "fft_reg.h"
+#include "fft_yz.h"
 
 using namespace amdk;
 
@@ -521,16 +521,241 @@ static void launch_z_rho(amdk_ctx* c, const Sphere& S, int np, double* rho, int 
   prof_end(c, ps);
 }
 
+// ---------------------------------------------------------------------------
+// the y-z kernels of fft_yz.h
+template <typename K>
+static void allow_lds(K kern, size_t lds) {
+  if (lds > 64 * 1024)
+    AMDK_TRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+}
+
+// Half rows per block of the transposing x passes: 16 (FP32) or 8 (FP64)
+// consecutive slots per x are one 128-byte run of W1.
+// The forward pass of the longer rows takes 8: its blocks of 16 leave too few
+// waves on a CU (144^3, 256 bands: 0.34 against 0.27 ms; 100^3, 128 bands: 16
+// 0.053, 8 0.059 ms).
+template <typename T> struct YzRows {
+  static constexpr int HR = sizeof(T) == 4 ? 16 : 8;
+  static constexpr int fwd(int tm) { return tm <= 10 ? HR : 8; }
+};
+
+template <typename T>
+static YzCols yz_cols(const Sphere& S) {
+  constexpr int q = YzRows<T>::HR;
+  YzCols k;
+  k.nrow = S.nrow;
+  k.base = (S.nrow + q - 1) / q * q;
+  k.pitch = k.base + k.base;
+  return k;
+}
+
+// What the y-z kernels need of a context: LDS bytes and resident blocks of
+// H|psi> and of the density, lane-order values and the lane order.
+struct YzPlan {
+  size_t lds_v = 0, lds_r = 0, native = 0;
+  int resident_v = 0, resident_r = 0, zs = 1;
+  double lanes = 0;
+  YzOrder order{};
+};
+template <typename T, int A, int B>
+static YzPlan yz_plan_ab(const amdk_ctx* c, const Sphere& S) {
+  using Y = YzShape<T, A, B>;
+  YzPlan p;
+  p.lds_v = Y::lds(S.nplane, Y::WV);
+  p.lds_r = Y::lds(S.nplane, Y::WR);
+  p.native = Y::native(c->n1);
+  // blocks in flight on 256 CUs: LDS, and registers for 16 waves per CU
+  p.resident_v = 256 * std::max(1, (int)std::min<size_t>(LDS_PER_CU / p.lds_v, 16 / Y::WV));
+  p.resident_r = 256 * std::max(1, (int)std::min<size_t>(LDS_PER_CU / p.lds_r, 16 / Y::WR));
+  p.zs = Y::ZS;
+  p.lanes = Y::lanes;
+  p.order = YzOrder{c->n1, Y::N, A, B, Y::TM, Y::CPW, Y::GZ};
+  return p;
+}
+template <typename T>
+static YzPlan yz_plan(const amdk_ctx* c, const Sphere& S) {
+  switch (c->n2) {
+#define AMDK_C(N, A, B) case N: return yz_plan_ab<T, A, B>(c, S);
+    AMDK_REG_SIZES(AMDK_C)
+#undef AMDK_C
+    default: return YzPlan{};
+  }
+}
+
+// Where the y-z kernels are used: a square y-z plane of a register length, a
+// sphere of consecutive rows within a quarter of the grid, LDS room for the
+// plane, and a length at which they measured faster than the separate passes
+// (96 bands, 70 Ry, both forms in turn; passes / y-z kernels).
+// H|psi> by itself gains wherever the transform fills a wave's lanes: 1.43 at
+// 100^3, 1.33 at 108^3, 1.26 at 144^3 in FP32, 1.60 and 1.38 at 100^3 and 108^3
+// in FP64; with fewer lanes busy (50 = 10 x 5, 60 = 10 x 6, 128 = 16 x 8)
+// 0.84-1.0, but below 40 the two launches saved count for more (1.27 at 32^3),
+// and from 150 on the planes' traffic.
+static bool yz_gains_vpsi(const YzPlan& p, int n) { return n < 40 || n >= 150 || p.lanes >= 0.78; }
+// An SCF step also takes the density from them and saves the separate passes'
+// second use of the planes: 1.04 at 100^3, 1.06 at 90^3 in FP32 and 1.11, 1.07
+// and 1.06 (108^3) in FP64, but 0.92 at 108^3 in FP32 (9 of 12 lanes) and
+// 0.92-0.98 for the smaller grids, whose planes the caches hold.  At 180^3
+// (12 of 15 lanes) 0.98 with 96 bands and 1.04 with 512.
+static bool yz_gains_scf(const YzPlan& p, int n, bool f64) {
+  return f64 ? n >= 90 && p.lanes >= 0.8 : n >= 72 && (p.lanes >= 0.88 || (n >= 180 && p.lanes >= 0.8));
+}
+// With few pairs in flight the density's pair groups do not fill the device
+// (16 pairs at 100^3: 0.111 against 0.103 ms).
+static bool use_yz_scf(const amdk_ctx* c, int npairs) { return c->yz_scf && npairs >= (c->n2 >= 150 ? 128 : 32); }
+
+template <typename T>
+static bool yz_fits(const amdk_ctx* c, const Sphere& S) {
+  if (c->n2 != c->n3 || !reg_ok(c, c->n1) || !reg_ok(c, c->n2) || !S.planes_contiguous) return false;
+  if (!quarter_z(S, c->n3) || !quarter_y(S, c->n2)) return false;
+  const YzPlan p = yz_plan<T>(c, S);
+  return p.lds_v <= LDS_PER_CU && p.lds_r <= LDS_PER_CU;
+}
+
+// Pair groups of the density: the count whose blocks fill the device in the
+// fewest rounds of pairs (the first such; a group's own cost, its grid
+// written and summed, counts as one pair).
+static int yz_rho_groups(const YzPlan& p, int n1, int npairs) {
+  int best = 1;
+  double best_cost = 1e300;
+  for (int g = 1; g <= std::min(npairs, 16); ++g) {
+    const int rounds = (n1 * p.zs * g + p.resident_r - 1) / p.resident_r;
+    const double cost = (double)rounds * ((npairs + g - 1) / g + 1);
+    if (cost < best_cost) { best_cost = cost; best = g; }
+  }
+  return best;
+}
+
+template <typename T, int A, int B>
+static void yz_vpsi_ab(amdk_ctx* c, const Sphere& S, int np, const YzPlan& p) {
+  using V = typename cplx_of<T>::type;
+  using Y = YzShape<T, A, B>;
+  allow_lds(k_yz_vpsi<T, A, B>, p.lds_v);
+  // pairs per block: as many as leave four rounds of blocks
+  const int PG = std::max(1, std::min(8, (int)((long)c->n1 * np / (4L * p.resident_v))));
+  const int ngrp = (np + PG - 1) / PG, per = (c->n1 * ngrp + 7) / 8;
+  k_yz_vpsi<T, A, B><<<8 * per, 64 * Y::WV, p.lds_v, c->stream>>>(geom_of(c, S), (V*)c->W1, yz_cols<T>(S), c->d_planes, (const T*)c->vn, np, PG,
+                                                              (const V*)(sizeof(T) == 4 ? c->tw_f[2] : c->tw_d[2]), ngrp, per);
+}
+template <typename T, int A, int B>
+static void yz_rho_ab(amdk_ctx* c, const Sphere& S, int np, const YzPlan& p, const double* wpair, int accumulate) {
+  using V = typename cplx_of<T>::type;
+  using Y = YzShape<T, A, B>;
+  allow_lds(k_yz_rho<T, A, B>, p.lds_r);
+  const int per = (c->n1 * Y::ZS * c->rho_groups + 7) / 8;
+  k_yz_rho<T, A, B><<<8 * per, 64 * Y::WR, p.lds_r, c->stream>>>(geom_of(c, S), (const V*)c->W1, yz_cols<T>(S), c->d_planes, c->d_rhopart, p.native,
+                                                             np, wpair, accumulate,
+                                                             (const V*)(sizeof(T) == 4 ? c->tw_f[2] : c->tw_d[2]),
+                                                             c->rho_groups, per);
+}
+template <typename T, int A, int B>
+static void yz_rows_inv_ab(amdk_ctx* c, const Sphere& S, const void* C, int nb, int pair0, int np) {
+  using V = typename cplx_of<T>::type;
+  constexpr int N = A * B, TM = MaxAB<A, B>::v, HR = YzRows<T>::HR;
+  const size_t lds = (size_t)(N + 2 * HR * (N + 1)) * sizeof(V);
+  allow_lds(k_rows_inv_t<T, A, B, HR>, lds);
+  k_rows_inv_t<T, A, B, HR><<<dim3((S.nrow + HR - 1) / HR, np), 2 * HR * TM, lds, c->stream>>>(
+      geom_of(c, S), (const double2*)C, S.ldc, nb, pair0, (V*)c->W1, yz_cols<T>(S),
+      (const V*)(sizeof(T) == 4 ? c->tw_f[0] : c->tw_d[0]));
+}
+template <typename T, int A, int B>
+static void yz_rows_fwd_ab(amdk_ctx* c, const Sphere& S, const void* C, void* C2, int nb, int pair0, int np) {
+  using V = typename cplx_of<T>::type;
+  constexpr int N = A * B, TM = MaxAB<A, B>::v, HR = YzRows<T>::fwd(TM);
+  const size_t lds = (size_t)(N + 2 * HR * (N + 1)) * sizeof(V);
+  allow_lds(k_rows_fwd_hpsi_t<T, A, B, HR>, lds);
+  k_rows_fwd_hpsi_t<T, A, B, HR><<<dim3((S.nrow + HR - 1) / HR, np), 2 * HR * TM, lds, c->stream>>>(
+      geom_of(c, S), (const V*)c->W1, yz_cols<T>(S), (const double2*)C, (double2*)C2, S.ldc, nb, pair0, c->d_occ, c->rc,
+      (const V*)(sizeof(T) == 4 ? c->tw_f[0] : c->tw_d[0]));
+}
+
+template <typename T>
+static void launch_yz_rows_inv(amdk_ctx* c, const Sphere& S, const void* C, int nb, int pair0, int np) {
+  const int ps = prof_begin(c, "rows_inv");
+  switch (c->n1) {
+#define AMDK_C(N, A, B) case N: yz_rows_inv_ab<T, A, B>(c, S, C, nb, pair0, np); break;
+    AMDK_REG_SIZES(AMDK_C)
+#undef AMDK_C
+  }
+  AMDK_TRY_HIP(hipGetLastError());
+  prof_end(c, ps);
+}
+template <typename T>
+static void launch_yz_rows_fwd(amdk_ctx* c, const Sphere& S, const void* C, void* C2, int nb, int pair0, int np) {
+  const int ps = prof_begin(c, "rows_fwd_hpsi");
+  switch (c->n1) {
+#define AMDK_C(N, A, B) case N: yz_rows_fwd_ab<T, A, B>(c, S, C, C2, nb, pair0, np); break;
+    AMDK_REG_SIZES(AMDK_C)
+#undef AMDK_C
+  }
+  AMDK_TRY_HIP(hipGetLastError());
+  prof_end(c, ps);
+}
+template <typename T>
+static void launch_yz_vpsi(amdk_ctx* c, const Sphere& S, int np) {
+  const YzPlan p = yz_plan<T>(c, S);
+  const int ps = prof_begin(c, "yz_vpsi");
+  switch (c->n2) {
+#define AMDK_C(N, A, B) case N: yz_vpsi_ab<T, A, B>(c, S, np, p); break;
+    AMDK_REG_SIZES(AMDK_C)
+#undef AMDK_C
+  }
+  AMDK_TRY_HIP(hipGetLastError());
+  prof_end(c, ps);
+}
+template <typename T>
+static void launch_yz_rho(amdk_ctx* c, const Sphere& S, int np, const double* wpair, int accumulate) {
+  const YzPlan p = yz_plan<T>(c, S);
+  const int ps = prof_begin(c, "yz_rho");
+  switch (c->n2) {
+#define AMDK_C(N, A, B) case N: yz_rho_ab<T, A, B>(c, S, np, p, wpair, accumulate); break;
+    AMDK_REG_SIZES(AMDK_C)
+#undef AMDK_C
+  }
+  AMDK_TRY_HIP(hipGetLastError());
+  prof_end(c, ps);
+}
+// V(r)/N of H|psi> from the dense FP64 grid v, in the lane order of the y-z
+// kernels (native) or x fastest
+template <typename T>
+static void launch_potential(amdk_ctx* c, const double* v, double scale, bool native) {
+  if (native) {
+    k_yz_potential<double, T><<<RED_BLOCKS, 256, 0, c->stream>>>(yz_plan<T>(c, c->spw).order, v, scale, (T*)c->vn);
+  } else {
+    const size_t nr = (size_t)c->n1 * c->n2 * c->n3;
+    k_scale_copy<T><<<1024, 256, 0, c->stream>>>(v, (T*)c->vr, nr, scale);
+  }
+  AMDK_TRY_HIP(hipGetLastError());
+  c->v_native = native;
+}
+// the potential of the last SCF step by separate passes, for an H|psi> by the
+// y-z kernels
+template <typename T>
+static void make_v_native(amdk_ctx* c) {
+  if (c->v_native) return;
+  k_yz_potential<T, T><<<RED_BLOCKS, 256, 0, c->stream>>>(yz_plan<T>(c, c->spw).order, (const T*)c->vr, 1.0, (T*)c->vn);
+  AMDK_TRY_HIP(hipGetLastError());
+  c->v_native = true;
+}
+
 template <typename T>
 // planes_ready: W2 already holds the y-transformed planes of all pairs of
-// these bands (left by run_density of the same C0 in one chunk), so the x and
-// y inverse passes are skipped.
+// these bands (use_yz_scf: W1 their rows), left by run_density of the same C0
+// in one chunk, so the inverse passes up to there are skipped.
 static void run_vpsi(amdk_ctx* c, const void* C0, void* C2, int nb, bool planes_ready = false) {
   const Sphere& S = c->spw;
   const int npairs = (nb + 1) / 2;
   if (planes_ready && npairs > c->cap_pairs) throw Error(AMDK_ERR_STATE, "planes of all pairs do not fit the work arrays");
+  const bool yz = planes_ready ? use_yz_scf(c, npairs) : c->yz_vpsi;
+  if (yz) make_v_native<T>(c);
   for (int p0 = 0; p0 < npairs; p0 += c->cap_pairs) {
     const int np = std::min(c->cap_pairs, npairs - p0);
+    if (yz) {
+      if (!planes_ready) launch_yz_rows_inv<T>(c, S, C0, nb, p0, np);
+      launch_yz_vpsi<T>(c, S, np);
+      launch_yz_rows_fwd<T>(c, S, C0, C2, nb, p0, np);
+      continue;
+    }
     if (!planes_ready) {
       launch_rows_inv<T>(c, S, C0, S.ldc, nb, p0, np);
       launch_cols<T>(c, S, np, true);
@@ -568,6 +793,20 @@ static void run_density(amdk_ctx* c, const void* C0, int nb, double* rho, bool n
   const Sphere& S = c->spw;
   const int npairs = (nb + 1) / 2;
   const size_t nr = (size_t)c->n1 * c->n2 * c->n3;
+  if (use_yz_scf(c, npairs)) {
+    for (int p0 = 0; p0 < npairs; p0 += c->cap_pairs) {
+      const int np = std::min(c->cap_pairs, npairs - p0);
+      launch_yz_rows_inv<T>(c, S, C0, nb, p0, np);
+      launch_yz_rho<T>(c, S, np, c->d_wpair + 2 * p0, p0 > 0);
+    }
+    const YzPlan p = yz_plan<T>(c, S);
+    k_yz_rho_combine<<<RED_BLOCKS, 256, 0, c->stream>>>(p.order, c->d_rhopart, p.native, c->rho_groups, rho,
+                                                       c->d_part + 8 * RED_BLOCKS);
+    AMDK_TRY_HIP(hipGetLastError());
+    if (norms_after) AMDK_TRY_HIP(hipStreamWaitEvent(c->stream, norms_after, 0));
+    if (sizeof(T) == 4) renormalise_density<T>(c, C0, nb, rho, norms_ready, true);
+    return;
+  }
   const bool grouped = rho == c->grid[0] && reg_ok(c, c->n3) && std::min(npairs, c->cap_pairs) >= 2 * RHO_GROUPS;
   for (int p0 = 0; p0 < npairs; p0 += c->cap_pairs) {
     const int np = std::min(c->cap_pairs, npairs - p0);
@@ -638,6 +877,7 @@ int amdk_ctx_create(const amdk_desc* d, amdk_ctx** out) {
     {
       const char* f = std::getenv("AMDK_FFT");
       ctx->fft_generic = f && std::string(f) == "stockham";
+      ctx->yz_vpsi = !(f && std::string(f) == "passes");
       const char* o = std::getenv("AMDK_OVL_BIG");
       ctx->ovl_big = !(o && std::string(o) == "0");
     }
@@ -712,13 +952,22 @@ int amdk_ctx_create(const amdk_desc* d, amdk_ctx** out) {
       upload(ctx, ctx->tw_f[ax], tf.data(), sizeof(float2) * n);
     }
     const size_t nr = (size_t)d->n1 * d->n2 * d->n3;
-    ctx->vr = dev_alloc(ctx, (ctx->prec == AMDK_PREC_FP64 ? sizeof(double) : sizeof(float)) * nr);
+    const bool f64 = ctx->prec == AMDK_PREC_FP64;
+    const bool fits = ctx->yz_vpsi && (f64 ? yz_fits<double>(ctx, ctx->spw) : yz_fits<float>(ctx, ctx->spw));
+    const YzPlan yzp = !fits ? YzPlan{} : f64 ? yz_plan<double>(ctx, ctx->spw) : yz_plan<float>(ctx, ctx->spw);
+    ctx->yz_vpsi = fits && yz_gains_vpsi(yzp, d->n2);
+    ctx->yz_scf = ctx->yz_vpsi && yz_gains_scf(yzp, d->n2, f64);
+    const size_t tb = f64 ? sizeof(double) : sizeof(float);
+    ctx->vr = dev_alloc(ctx, tb * nr);
+    if (ctx->yz_vpsi) ctx->vn = dev_alloc(ctx, tb * yzp.native);
     // FFT work arrays for up to cap_pairs band pairs at once (W1 + W2 within
     // 24 GiB of the 288 GiB of HBM3E; AMDK_PAIR_BUDGET_MB overrides it, e.g.
     // to exercise the chunked path at small sizes)
     const Sphere& S = ctx->spw;
     const size_t w2_pair = (size_t)S.nplane * d->n2 * row_pitch(d->n1) * cbytes(ctx);
-    const size_t w1_pair = (size_t)S.nslot * row_pitch(d->n1) * cbytes(ctx);
+    size_t w1_pair = (size_t)S.nslot * row_pitch(d->n1) * cbytes(ctx);
+    if (ctx->yz_vpsi)
+      w1_pair = std::max(w1_pair, (size_t)d->n1 * (f64 ? yz_cols<double>(S) : yz_cols<float>(S)).pitch * cbytes(ctx));
     const int npairs = (d->nbmax + 1) / 2;
     size_t budget = (size_t)24 << 30;
     if (const char* b = std::getenv("AMDK_PAIR_BUDGET_MB")) {
@@ -728,6 +977,20 @@ int amdk_ctx_create(const amdk_desc* d, amdk_ctx** out) {
     ctx->cap_pairs = (int)std::max<size_t>(1, std::min<size_t>(npairs, budget / (w2_pair + w1_pair)));
     ctx->W1 = dev_alloc(ctx, w1_pair * ctx->cap_pairs);
     ctx->W2 = dev_alloc(ctx, w2_pair * ctx->cap_pairs);
+    if (ctx->yz_vpsi) {
+      const YzCols cols = f64 ? yz_cols<double>(S) : yz_cols<float>(S);
+      std::vector<int4> planes(S.nplane);
+      for (int p = 0; p < S.nplane; ++p) {
+        const int s0 = S.h_plane_off[p], s1 = S.h_plane_off[p + 1];
+        planes[p] = cols.plane(s0, s1, s1 > s0 ? S.h_slot_m2[s0] : 0);
+      }
+      ctx->d_planes = (int4*)dev_alloc(ctx, sizeof(int4) * S.nplane);
+      upload(ctx, ctx->d_planes, planes.data(), sizeof(int4) * S.nplane);
+    }
+    if (ctx->yz_scf) {
+      ctx->rho_groups = yz_rho_groups(yzp, d->n1, ctx->cap_pairs);
+      ctx->d_rhopart = (double*)dev_alloc(ctx, sizeof(double) * yzp.native * ctx->rho_groups);
+    }
     ctx->d_occ = (double*)dev_alloc(ctx, sizeof(double) * (d->nbmax + 1));
     ctx->d_wpair = (double*)dev_alloc(ctx, sizeof(double) * (d->nbmax + 2));
     ctx->d_wdens = (double*)dev_alloc(ctx, sizeof(double) * (d->nbmax + 1));
@@ -782,11 +1045,8 @@ int amdk_set_vks(amdk_ctx* ctx, const double* v_r) {
   double* stage = ctx->grid[1];  // dense scratch grid, free between calls
   grid_in(ctx, v_r, stage);
   const double s = 1.0 / (double)nr;  // forward FFT normalisation folded into V
-  if (ctx->prec == AMDK_PREC_FP64)
-    k_scale_copy<double><<<1024, 256, 0, ctx->stream>>>(stage, (double*)ctx->vr, nr, s);
-  else
-    k_scale_copy<float><<<1024, 256, 0, ctx->stream>>>(stage, (float*)ctx->vr, nr, s);
-  AMDK_TRY_HIP(hipGetLastError());
+  if (ctx->prec == AMDK_PREC_FP64) launch_potential<double>(ctx, stage, s, ctx->yz_vpsi);
+  else launch_potential<float>(ctx, stage, s, ctx->yz_vpsi);
   AMDK_TRY_HIP(hipStreamSynchronize(ctx->stream));
   ctx->have_vks = true;
   API_END

@@ -63,13 +63,22 @@ struct amdk_ctx {
   // twiddles exp(-2 pi i t/n) in float2 and double2
   void* tw_f[3] = {nullptr, nullptr, nullptr};
   void* tw_d[3] = {nullptr, nullptr, nullptr};
-  // V_KS(r)/N in the compute precision; set flag
+  // V_KS(r)/N in the compute precision, x fastest (vr) and in the lane order of
+  // fft_yz.h (vn); v_native: vn holds it, otherwise vr; set flag
   void* vr = nullptr;
+  void* vn = nullptr;
+  bool v_native = false;
   bool have_vks = false;
   // FFT workspaces sized for `cap_pairs` band pairs
   void* W1 = nullptr;
-  void* W2 = nullptr;
+  void* W2 = nullptr;         // planes of the separate passes
   int cap_pairs = 0;
+  // y and z transforms in one kernel (fft_yz.h; W1 then transposed): for H|psi>
+  // by itself, and for the density with what follows it in an SCF step
+  bool yz_vpsi = false, yz_scf = false;
+  int4* d_planes = nullptr;   // rows of each plane (YzCols::plane)
+  double* d_rhopart = nullptr;
+  int rho_groups = 1;
   double* d_occ = nullptr;   // [nbmax]
   double* d_wpair = nullptr; // [nbmax+1]
   // internal Miller indices (3 ints per G) of both spheres

@@ -32,76 +32,122 @@ __device__ __forceinline__ V csub(V a, V b) { V r; r.x = a.x - b.x; r.y = a.y - 
 template <int S, typename V>
 __device__ __forceinline__ V mul_si(V a) { V r; r.x = -S * a.y; r.y = S * a.x; return r; }
 
-template <typename V, int R, int DIR> struct Butterfly;
+// sums of two values of which ZA or ZB says that it is 0 and not to be read
+template <bool ZA, bool ZB, typename V>
+__device__ __forceinline__ V cadd_z(V a, V b) {
+  if constexpr (ZA) return b;
+  else if constexpr (ZB) return a;
+  else return cadd(a, b);
+}
+template <bool ZA, bool ZB, typename V>
+__device__ __forceinline__ V csub_z(V a, V b) {
+  if constexpr (ZA) { b.x = -b.x; b.y = -b.y; return b; }
+  else if constexpr (ZB) return a;
+  else return csub(a, b);
+}
 
-template <typename V, int DIR> struct Butterfly<V, 2, DIR> {
+// R-point DFT in place; bit j of Z says that v[j] is 0 and not to be read
+// (fewer than all).
+template <typename V, int R, int DIR, unsigned Z = 0> struct Butterfly;
+
+template <typename V, int DIR, unsigned Z> struct Butterfly<V, 2, DIR, Z> {
   __device__ static __forceinline__ void run(V* v) {
+    constexpr bool z0 = Z & 1, z1 = Z & 2;
     V a = v[0], b = v[1];
-    v[0] = cadd(a, b);
-    v[1] = csub(a, b);
+    v[0] = cadd_z<z0, z1>(a, b);
+    v[1] = csub_z<z0, z1>(a, b);
   }
 };
 
-template <typename V, int DIR> struct Butterfly<V, 3, DIR> {
+template <typename V, int DIR, unsigned Z> struct Butterfly<V, 3, DIR, Z> {
   __device__ static __forceinline__ void run(V* v) {
     using T = decltype(v[0].x);
+    constexpr bool z0 = Z & 1, z1 = Z & 2, z2 = Z & 4;
     const T h = (T)0.86602540378443864676;  // sqrt(3)/2
-    V t = cadd(v[1], v[2]);
-    V d = mul_si<DIR>(csub(v[1], v[2]));
     V a0 = v[0];
-    V m;  // a0 - t/2
-    m.x = a0.x - (T)0.5 * t.x;
-    m.y = a0.y - (T)0.5 * t.y;
-    v[0] = cadd(a0, t);
-    v[1].x = m.x + h * d.x;
-    v[1].y = m.y + h * d.y;
-    v[2].x = m.x - h * d.x;
-    v[2].y = m.y - h * d.y;
+    if constexpr (z1 && z2) {
+      v[1] = v[2] = a0;
+    } else {
+      V t = cadd_z<z1, z2>(v[1], v[2]);
+      V d = mul_si<DIR>(csub_z<z1, z2>(v[1], v[2]));
+      V m;  // a0 - t/2
+      if constexpr (z0) {
+        m.x = (T)-0.5 * t.x;
+        m.y = (T)-0.5 * t.y;
+      } else {
+        m.x = a0.x - (T)0.5 * t.x;
+        m.y = a0.y - (T)0.5 * t.y;
+      }
+      v[0] = cadd_z<z0, false>(a0, t);
+      v[1].x = m.x + h * d.x;
+      v[1].y = m.y + h * d.y;
+      v[2].x = m.x - h * d.x;
+      v[2].y = m.y - h * d.y;
+    }
   }
 };
 
-template <typename V, int DIR> struct Butterfly<V, 4, DIR> {
+template <typename V, int DIR, unsigned Z> struct Butterfly<V, 4, DIR, Z> {
   __device__ static __forceinline__ void run(V* v) {
-    V t0 = cadd(v[0], v[2]);
-    V t1 = csub(v[0], v[2]);
-    V t2 = cadd(v[1], v[3]);
-    V t3 = mul_si<DIR>(csub(v[1], v[3]));
-    v[0] = cadd(t0, t2);
-    v[2] = csub(t0, t2);
-    v[1] = cadd(t1, t3);
-    v[3] = csub(t1, t3);
+    constexpr bool z0 = Z & 1, z1 = Z & 2, z2 = Z & 4, z3 = Z & 8;
+    V t0 = cadd_z<z0, z2>(v[0], v[2]);
+    V t1 = csub_z<z0, z2>(v[0], v[2]);
+    V t2 = cadd_z<z1, z3>(v[1], v[3]);
+    V t3 = mul_si<DIR>(csub_z<z1, z3>(v[1], v[3]));
+    constexpr bool ze = z0 && z2, zo = z1 && z3;
+    v[0] = cadd_z<ze, zo>(t0, t2);
+    v[2] = csub_z<ze, zo>(t0, t2);
+    v[1] = cadd_z<ze, zo>(t1, t3);
+    v[3] = csub_z<ze, zo>(t1, t3);
   }
 };
 
-template <typename V, int DIR> struct Butterfly<V, 5, DIR> {
+template <typename V, int DIR, unsigned Z> struct Butterfly<V, 5, DIR, Z> {
   __device__ static __forceinline__ void run(V* v) {
     using T = decltype(v[0].x);
+    constexpr bool z0 = Z & 1, z1 = Z & 2, z2 = Z & 4, z3 = Z & 8, z4 = Z & 16;
+    constexpr bool zo = z1 && z4, zi = z2 && z3;  // outer and inner pair
     const T c1 = (T)0.30901699437494742410;   // cos(2pi/5)
     const T c2 = (T)-0.80901699437494742410;  // cos(4pi/5)
     const T s1 = (T)0.95105651629515357212;   // sin(2pi/5)
     const T s2 = (T)0.58778525229247312917;   // sin(4pi/5)
     V a0 = v[0];
-    V t1 = cadd(v[1], v[4]);
-    V t2 = cadd(v[2], v[3]);
-    V t3 = csub(v[1], v[4]);
-    V t4 = csub(v[2], v[3]);
-    V b1, b2, e1, e2;
-    b1.x = a0.x + c1 * t1.x + c2 * t2.x;
-    b1.y = a0.y + c1 * t1.y + c2 * t2.y;
-    b2.x = a0.x + c2 * t1.x + c1 * t2.x;
-    b2.y = a0.y + c2 * t1.y + c1 * t2.y;
-    e1.x = s1 * t3.x + s2 * t4.x;
-    e1.y = s1 * t3.y + s2 * t4.y;
-    e2.x = s2 * t3.x - s1 * t4.x;
-    e2.y = s2 * t3.y - s1 * t4.y;
-    V d1 = mul_si<DIR>(e1);
-    V d2 = mul_si<DIR>(e2);
-    v[0].x = a0.x + t1.x + t2.x;
-    v[0].y = a0.y + t1.y + t2.y;
-    v[1] = cadd(b1, d1);
-    v[4] = csub(b1, d1);
-    v[2] = cadd(b2, d2);
-    v[3] = csub(b2, d2);
+    if constexpr (zo && zi) {
+      v[1] = v[2] = v[3] = v[4] = a0;
+    } else {
+      V t1 = cadd_z<z1, z4>(v[1], v[4]);
+      V t2 = cadd_z<z2, z3>(v[2], v[3]);
+      V t3 = csub_z<z1, z4>(v[1], v[4]);
+      V t4 = csub_z<z2, z3>(v[2], v[3]);
+      // a0 + p t1 + q t2 and p t3 + q t4 without the terms that are 0
+      auto even = [&](T x0, T p, T x1, T q, T x2) {
+        if constexpr (zi) return z0 ? p * x1 : x0 + p * x1;
+        else if constexpr (zo) return z0 ? q * x2 : x0 + q * x2;
+        else if constexpr (z0) return p * x1 + q * x2;
+        else return x0 + p * x1 + q * x2;
+      };
+      auto odd = [&](T p, T x3, T q, T x4) {
+        if constexpr (zi) return p * x3;
+        else if constexpr (zo) return q * x4;
+        else return p * x3 + q * x4;
+      };
+      V b1, b2, e1, e2;
+      b1.x = even(a0.x, c1, t1.x, c2, t2.x);
+      b1.y = even(a0.y, c1, t1.y, c2, t2.y);
+      b2.x = even(a0.x, c2, t1.x, c1, t2.x);
+      b2.y = even(a0.y, c2, t1.y, c1, t2.y);
+      e1.x = odd(s1, t3.x, s2, t4.x);
+      e1.y = odd(s1, t3.y, s2, t4.y);
+      e2.x = odd(s2, t3.x, -s1, t4.x);
+      e2.y = odd(s2, t3.y, -s1, t4.y);
+      V d1 = mul_si<DIR>(e1);
+      V d2 = mul_si<DIR>(e2);
+      v[0] = cadd_z<z0 && zo, zi>(cadd_z<z0, zo>(a0, t1), t2);
+      v[1] = cadd(b1, d1);
+      v[4] = csub(b1, d1);
+      v[2] = cadd(b2, d2);
+      v[3] = csub(b2, d2);
+    }
   }
 };
 

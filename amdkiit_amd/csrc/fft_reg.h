@@ -53,32 +53,52 @@ __device__ __forceinline__ V mul_root(V a, int m) {
 // fewer vector instructions and rounds less (FP32 H|psi> at 100^3 against 64
 // bits: 1.05e-8 -> 8.2e-9): z_vpsi 0.172 -> 0.168 ms at 32 H2O, 0.817 ->
 // 0.797 ms at 64 H2O.
-template <typename V, int L, int DIR> struct RDft {
+// Z: bit j set says that x[j] is 0 (and not to be read); the sums and products
+// with it are left out, which changes no result.
+template <typename V, int L, int DIR, unsigned Z = 0> struct RDft {
+  static constexpr int P = Split<L>::P, Q = Split<L>::Q;
+  static constexpr bool PF = gcd_of(P, Q) == 1;
+  static constexpr int in_of(int k1, int k2) { return PF ? (Q * k1 + P * k2) % L : k1 + P * k2; }
+  static constexpr unsigned zeros_of(int k1) {  // of the Q-point DFT k1
+    unsigned z = 0;
+    for (int k2 = 0; k2 < Q; ++k2)
+      if ((Z >> in_of(k1, k2)) & 1u) z |= 1u << k2;
+    return z;
+  }
+  static constexpr unsigned zeros_outer() {  // Q-point DFTs that are 0
+    unsigned z = 0;
+    for (int k1 = 0; k1 < P; ++k1)
+      if (zeros_of(k1) == (1u << Q) - 1u) z |= 1u << k1;
+    return z;
+  }
+  template <int K1> __device__ static __forceinline__ void inner(const V* x, V* y) {
+    if constexpr (K1 < P) {
+      if constexpr (zeros_of(K1) != (1u << Q) - 1u) {
+        V t[Q];
+#pragma unroll
+        for (int k2 = 0; k2 < Q; ++k2) t[k2] = x[in_of(K1, k2)];
+        RDft<V, Q, DIR, zeros_of(K1)>::run(t);
+#pragma unroll
+        for (int j2 = 0; j2 < Q; ++j2) y[K1 * Q + j2] = PF ? t[j2] : mul_root<L, DIR>(t[j2], (j2 * K1) % L);
+      }
+      inner<K1 + 1>(x, y);
+    }
+  }
   __device__ static __forceinline__ void run(V* x) {
     if constexpr (L == 1) {
       return;
     } else if constexpr (L <= 5) {
-      Butterfly<V, L, DIR>::run(x);
+      Butterfly<V, L, DIR, Z>::run(x);
     } else {
-      constexpr int P = Split<L>::P, Q = Split<L>::Q;
       static_assert(P * Q == L && P > 1, "no split for this DFT length");
-      constexpr bool PF = gcd_of(P, Q) == 1;
       V y[L];
-#pragma unroll
-      for (int k1 = 0; k1 < P; ++k1) {
-        V t[Q];
-#pragma unroll
-        for (int k2 = 0; k2 < Q; ++k2) t[k2] = x[PF ? (Q * k1 + P * k2) % L : k1 + P * k2];
-        RDft<V, Q, DIR>::run(t);
-#pragma unroll
-        for (int j2 = 0; j2 < Q; ++j2) y[k1 * Q + j2] = PF ? t[j2] : mul_root<L, DIR>(t[j2], (j2 * k1) % L);
-      }
+      inner<0>(x, y);
 #pragma unroll
       for (int j2 = 0; j2 < Q; ++j2) {
         V u[P];
 #pragma unroll
         for (int k1 = 0; k1 < P; ++k1) u[k1] = y[k1 * Q + j2];
-        RDft<V, P, DIR>::run(u);
+        RDft<V, P, DIR, zeros_outer()>::run(u);
 #pragma unroll
         for (int j1 = 0; j1 < P; ++j1) {
           if constexpr (PF) {
@@ -102,10 +122,11 @@ template <int A, int B> struct MaxAB { static constexpr int v = A > B ? A : B; }
 // Out: thread t < B holds X[t + B*j1], j1 < A, in r[0..A).
 // lds: A*B*stride elements; element (k1, j2) of column c at (k1*B + j2)*stride + c*cstride.
 // twN[m] = exp(-2 pi i m / N).  Every thread of the block must call this.
-template <typename V, int A, int B, int DIR>
+// Z: inputs that are 0 in every thread, as in RDft.
+template <typename V, int A, int B, int DIR, unsigned Z = 0>
 __device__ __forceinline__ void col_fft(V* r, int t, V* lds, int stride, int coff, const V* twN) {
   if (t < A) {
-    RDft<V, B, DIR>::run(r);
+    RDft<V, B, DIR, Z>::run(r);
 #pragma unroll
     for (int j2 = 0; j2 < B; ++j2) {
       V v = r[j2];
@@ -182,6 +203,15 @@ constexpr bool pencil_run(int k) {
   return !QW || 4 * A * k <= N || 4 * (N - A * k - A + 1) <= N;
 }
 
+// the runs that pencil_run leaves out, as the zeros of the length-B DFT over k
+template <bool QW, int A, int B>
+constexpr unsigned pencil_zeros() {
+  unsigned z = 0;
+  for (int k = 0; k < B; ++k)
+    if (!pencil_run<QW, A, A * B>(k)) z |= 1u << k;
+  return z;
+}
+
 // Block order of the z passes: MI355X hands consecutive workgroups
 // round-robin to its 8 XCDs; physical block p runs logical block
 // (p % 8) * per + p / 8, so each XCD walks one contiguous range of logical
@@ -238,7 +268,7 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
       if (pencil_run<QW, A, N>(k2)) r[k2] = buf.load(base + pencil_step<A, N>(t, k2) * psb);
       else r[k2].x = r[k2].y = 0;
     }
-    col_fft<V, A, B, +1>(r, t, lds, TX, c, tw);
+    col_fft<V, A, B, +1, pencil_zeros<QW, A, B>()>(r, t, lds, TX, c, tw);
     if (t < B) {
 #pragma unroll
       for (int j1 = 0; j1 < A; ++j1) {
@@ -306,7 +336,7 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
     } else {
       load_pair(pl, r);
     }
-    col_fft<V, A, B, +1>(r, t, lds, TX, c, tw);
+    col_fft<V, A, B, +1, pencil_zeros<QW, A, B>()>(r, t, lds, TX, c, tw);
     const double w1 = wpair[2 * pl], w2 = wpair[2 * pl + 1];
 #pragma unroll
     for (int j1 = 0; j1 < A; ++j1) {
@@ -352,7 +382,7 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
     if (pencil_run<QW, A, N>(k2)) r[k2] = rows.load(base + pencil_step<A, N>(t, k2) * psb);
     else r[k2].x = r[k2].y = 0;
   }
-  col_fft<V, A, B, +1>(r, t, lds, TX, c, tw);
+  col_fft<V, A, B, +1, pencil_zeros<QW, A, B>()>(r, t, lds, TX, c, tw);
   if (t < B && live) {
     V* out = W2 + ((size_t)pl * g.nplane + plane) * (size_t)n2 * g.p1 + (size_t)t * g.p1 + x;
 #pragma unroll

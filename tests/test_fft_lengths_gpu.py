@@ -1,7 +1,8 @@
 """H|psi> and the density at every transform length of the register passes
-that the other tests leave out (three at a time, one per axis), and with a
+that the other tests leave out: three at a time, one per axis (separate y and
+z passes), with equal y and z lengths (both in one kernel), and with a
 wavefunction sphere wider than a quarter of the grid, where no frequency run
-may be left out of the z and y passes."""
+may be left out."""
 import numpy as np
 import pytest
 
@@ -16,6 +17,10 @@ GRIDS = [(32, 40, 50), (54, 64, 80), (90, 96, 120), (128, 150, 20), (24, 160, 16
          (162, 128, 32), (50, 90, 64), (40, 54, 96), (64, 32, 90), (80, 48, 54), (96, 50, 40), (120, 80, 48), (150, 24, 60)]
 
 
+LENGTHS = (20, 24, 30, 32, 36, 40, 48, 50, 54, 60, 64, 72, 80, 90, 96, 100, 108, 120, 128, 144, 150, 160, 162, 180, 192)
+SQUARE = [(24, k, k) for k in LENGTHS] + [(k, 20, 20) for k in LENGTHS if k >= 32]
+
+
 def rel(a, b):
     return np.abs(a - b).max() / np.abs(b).max()
 
@@ -26,7 +31,7 @@ def sphere_to_the_edge(n):
 
 
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("mixed", 2e-6)])
-@pytest.mark.parametrize("n", GRIDS, ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("n", GRIDS + SQUARE, ids=lambda n: "x".join(map(str, n)))
 def test_lengths(n, prec, tol):
     pw = sphere_to_the_edge(n)
     nb = 3
@@ -57,3 +62,28 @@ def test_sphere_wider_than_a_quarter_of_the_grid(n, prec, tol):
     assert rel(ctx.vpsi(c, occ), O.vpsi(c, occ, v, pw.mill_pw, pw.n, pw.cell.g)) < tol
     assert rel(ctx.eval_density(c, occ), O.eval_density(c, occ, pw.mill_pw, pw.n, pw.cell.omega)) < tol
     ctx.close()
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("mixed", 2e-6)])
+@pytest.mark.parametrize("nb", [1, 2, 9, 33])
+def test_one_kernel_matches_separate_passes(nb, prec, tol, monkeypatch):
+    """The y-z kernels against the separate passes: pair groups and pairs per
+    block at several band counts, one pair chunk and several."""
+    pw = sphere_to_the_edge((30, 36, 36))
+    c = random_bands(pw, nb, seed=6)
+    occ = np.linspace(2.0, 0.0, nb)
+    v = smooth_potential(pw)
+    out = {}
+    for fft, budget in (("passes", None), ("", None), ("", "1")):
+        monkeypatch.setenv("AMDK_FFT", fft)
+        if budget:
+            monkeypatch.setenv("AMDK_PAIR_BUDGET_MB", budget)
+        print(f"case=one_kernel nb={nb} prec={prec} fft={fft!r} budget={budget}", flush=True)
+        ctx = KSContext(pw, nb, prec)
+        ctx.set_vks(v)
+        out[fft, budget] = (ctx.vpsi(c, occ), ctx.eval_density(c, occ))
+        ctx.close()
+    for key in (("", None), ("", "1")):
+        assert rel(out[key][0], out["passes", None][0]) < tol
+        assert rel(out[key][1], out["passes", None][1]) < tol
+    assert np.array_equal(out["", None][0], out["", "1"][0])
