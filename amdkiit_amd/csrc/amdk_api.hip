@@ -2,11 +2,13 @@
 // density drivers behind the C ABI declared in include/amdk.h.
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <numeric>
+#include <thread>
 #include <tuple>
 
 #include "amdk_ctx.h"
@@ -244,18 +246,153 @@ __global__ void k_scale_copy(const double* __restrict__ src, T* __restrict__ dst
     dst[i] = (T)(src[i] * s);
 }
 
+// Copies between a caller's (pageable) host array of `rows` rows of row_bytes,
+// `pitch` bytes apart, and a packed device array.  Into the device the
+// runtime's copy is used: it takes pageable memory at 27-30 GB/s, and workers
+// of our own gain a fifth on it at best and lose to the spinning threads of a
+// caller's parallel region (24 MB 0.93 -> 0.75 ms alone, 4 ms beside them).
+// The caller synchronises the stream before the host array can change.
+static void copy_in(amdk_ctx* c, void* dev, const void* host, size_t rows, size_t row_bytes, size_t pitch) {
+  AMDK_TRY_HIP(hipMemcpy2DAsync(dev, row_bytes, host, pitch, row_bytes, rows, hipMemcpyHostToDevice, c->stream));
+}
+
+// Out of the device the runtime's copy is one thread's (15-18 GB/s, first
+// touch of the caller's pages included), so the context's workers take 2 MiB
+// chunks through two pinned slots each, one moved to the caller's array while
+// the DMA fills the other: 64 H2O bands (320 MB) into new memory 31.5 -> 10.7
+// ms, 32 H2O (65 MB) 6.0 -> 2.1 ms.  Below COPY_MIN the plain copy stays:
+// starting the threads takes longer than they save.  The workers live for the
+// call; the calling thread is one of them and does all the work if no other
+// can be started.  Returns with the data in the caller's array.
+constexpr size_t COPY_SLOT = 2u << 20, COPY_MIN = 10u << 20;
+constexpr int COPY_WORKERS = 8;
+
+static void copy_setup(amdk_ctx* c, size_t largest) {
+  const int cpus = std::max(1, (int)std::thread::hardware_concurrency());
+  const int n = (int)std::min<size_t>(std::min(COPY_WORKERS, std::max(1, cpus / 2)), largest / (2 * COPY_SLOT));
+  if (n < 2 || largest < COPY_MIN) return;
+  AMDK_TRY_HIP(hipHostMalloc(&c->h_slots, 2 * COPY_SLOT * n, hipHostMallocDefault));
+  c->copy_ev.assign(2 * n, nullptr);
+  for (hipEvent_t& e : c->copy_ev) AMDK_TRY_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  c->copy_workers = n;
+}
+static void copy_destroy(amdk_ctx* c) {
+  for (hipEvent_t e : c->copy_ev)
+    if (e) (void)hipEventDestroy(e);
+  c->copy_ev.clear();
+  if (c->h_slots) (void)hipHostFree(c->h_slots);
+  c->h_slots = nullptr;
+  c->copy_workers = 0;
+}
+
+static void copy_out(amdk_ctx* c, const void* dev, void* host, size_t rows, size_t row_bytes, size_t pitch) {
+  const size_t total = rows * row_bytes;
+  if (total < COPY_MIN || c->copy_workers < 2) {
+    AMDK_TRY_HIP(hipMemcpy2DAsync(host, pitch, dev, row_bytes, row_bytes, rows, hipMemcpyDeviceToHost, c->stream));
+    AMDK_TRY_HIP(hipStreamSynchronize(c->stream));
+    return;
+  }
+  if (pitch == row_bytes) {  // one run
+    row_bytes = total;
+    rows = 1;
+  }
+  const size_t per_row = (row_bytes + COPY_SLOT - 1) / COPY_SLOT, nchunk = rows * per_row;
+  std::atomic<size_t> next{0};
+  std::atomic<int> err{(int)hipSuccess};
+  const int nw = (int)std::min<size_t>(c->copy_workers, total / (2 * COPY_SLOT));
+  struct Piece { char* h; const char* d; size_t n; };
+  auto work = [&](int w) noexcept {
+    auto ok = [&](hipError_t e) {
+      if (e != hipSuccess) err = (int)e;
+      return e == hipSuccess;
+    };
+    if (!ok(hipSetDevice(c->device))) return;
+    char* slot[2] = {c->h_slots + 2 * COPY_SLOT * w, c->h_slots + 2 * COPY_SLOT * w + COPY_SLOT};
+    const hipEvent_t ev[2] = {c->copy_ev[2 * w], c->copy_ev[2 * w + 1]};
+    auto fetch = [&](Piece& p, int s) {  // the next chunk into slot s; false: none left, or an error
+      if (err != (int)hipSuccess) return false;
+      const size_t k = next++;
+      if (k >= nchunk) return false;
+      const size_t r = k / per_row, o = (k % per_row) * COPY_SLOT;
+      p = {(char*)host + r * pitch + o, (const char*)dev + r * row_bytes + o, std::min(COPY_SLOT, row_bytes - o)};
+      return ok(hipMemcpyAsync(slot[s], p.d, p.n, hipMemcpyDeviceToHost, c->stream)) && ok(hipEventRecord(ev[s], c->stream));
+    };
+    Piece p[2];
+    bool have = fetch(p[0], 0);
+    for (int i = 0; have; ++i) {
+      const int s = i & 1;
+      have = fetch(p[s ^ 1], s ^ 1);
+      if (!ok(hipEventSynchronize(ev[s]))) return;
+      std::memcpy(p[s].h, slot[s], p[s].n);
+    }
+  };
+  {
+    struct Team {
+      std::vector<std::thread> t;
+      ~Team() {
+        for (auto& x : t) x.join();
+      }
+    } team;
+    try {
+      team.t.reserve(nw - 1);
+      for (int w = 1; w < nw; ++w) team.t.emplace_back(work, w);
+    } catch (const std::exception&) {
+      // fewer workers: the ones that run take all the chunks
+    }
+    work(0);
+  }
+  const hipError_t fin = hipStreamSynchronize(c->stream);  // no slot is in use after the call
+  if (err != (int)hipSuccess)
+    throw Error(AMDK_ERR_DEVICE, std::string("host copy: ") + hipGetErrorString((hipError_t)err.load()));
+  AMDK_TRY_HIP(fin);
+}
+
+// *flag = 1 if any of the n values is not finite.  Bound by memory; 2,048
+// blocks of independent loads (0.07 ms for 320 MB, on the host 9 ms).
+__global__ void __launch_bounds__(256) k_check_finite(const double* __restrict__ x, size_t n, int* __restrict__ flag) {
+  bool bad = false;
+  for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) bad |= !isfinite(x[i]);
+  if (bad) *flag = 1;
+}
+__global__ void k_clear_int(int* p) { *p = 0; }
+// Smaller arrays are checked on the host (33 GB/s; the device's answer takes
+// two launches and a copy, 0.03 ms).
+constexpr size_t DEV_CHECK_MIN = 1u << 20;
+
+static void check_finite(const double* p, size_t n, const char* what) {
+  for (size_t i = 0; i < n; ++i)
+    if (!std::isfinite(p[i])) throw Error(AMDK_ERR_NONFINITE, std::string("non-finite value in ") + what);
+}
+static void check_finite_dev(amdk_ctx* c, const void* p, size_t n, const char* what) {
+  k_clear_int<<<1, 1, 0, c->stream>>>(c->d_flag);
+  k_check_finite<<<2048, 256, 0, c->stream>>>((const double*)p, n, c->d_flag);
+  AMDK_TRY_HIP(hipGetLastError());
+  int bad = 0;
+  download(c, &bad, c->d_flag, sizeof(int));
+  if (bad) throw Error(AMDK_ERR_NONFINITE, std::string("non-finite value in ") + what);
+}
+
 // Caller-layout FP64 host arrays <-> internal device layout.  The caller's
-// first npw coefficients of each band are copied with their pitch into the
-// context's staging array (pitch ldc), then permuted on the device; nothing
-// is allocated per call.  Entries of the caller's array beyond npw are
-// neither read nor written.
-static void bands_in(amdk_ctx* c, const double* host, int ldsrc, int nb, void* dst) {
+// first npw coefficients of each band are copied into the context's staging
+// array (packed), then permuted on the device; nothing is allocated per call.
+// With `what`, values that are not finite are refused before dst is written:
+// also those in the caller's padding beyond npw, which is otherwise neither
+// read nor written.
+static void bands_in(amdk_ctx* c, const double* host, int ldsrc, int nb, void* dst, const char* what = nullptr) {
   const Sphere& S = c->spw;
-  AMDK_TRY_HIP(hipMemcpy2DAsync(c->d_stage, sizeof(double2) * S.ldc, host, sizeof(double2) * ldsrc,
-                                sizeof(double2) * S.npw, nb, hipMemcpyHostToDevice, c->stream));
+  const size_t row = sizeof(double2) * S.npw;
+  const bool small = row * nb < DEV_CHECK_MIN;
+  if (what && small) {
+    check_finite(host, (size_t)2 * ldsrc * nb, what);
+  } else if (what && ldsrc > S.npw) {
+    for (int b = 0; b < nb; ++b)
+      check_finite(host + 2 * ((size_t)b * ldsrc + S.npw), (size_t)2 * (ldsrc - S.npw), what);
+  }
+  copy_in(c, c->d_stage, host, nb, row, sizeof(double2) * ldsrc);
+  if (what && !small) check_finite_dev(c, c->d_stage, (size_t)2 * S.npw * nb, what);
   AMDK_TRY_HIP(hipMemsetAsync(dst, 0, sbytes(c) * (size_t)S.ldc * nb, c->stream));
   dim3 grid((S.npw + 255) / 256, nb);
-  k_from_caller<double2><<<grid, 256, 0, c->stream>>>((const double2*)c->d_stage, S.ldc, (double2*)dst, S.ldc,
+  k_from_caller<double2><<<grid, 256, 0, c->stream>>>((const double2*)c->d_stage, S.npw, (double2*)dst, S.ldc,
                                                       S.d_from_caller, S.d_conj_caller, S.npw, nb);
   AMDK_TRY_HIP(hipGetLastError());
   AMDK_TRY_HIP(hipStreamSynchronize(c->stream));
@@ -264,12 +401,10 @@ static void bands_in(amdk_ctx* c, const double* host, int ldsrc, int nb, void* d
 static void bands_out(amdk_ctx* c, const void* src, int nb, double* host, int lddst) {
   const Sphere& S = c->spw;
   dim3 grid((S.npw + 255) / 256, nb);
-  k_to_caller<double2><<<grid, 256, 0, c->stream>>>((const double2*)src, S.ldc, (double2*)c->d_stage, S.ldc,
+  k_to_caller<double2><<<grid, 256, 0, c->stream>>>((const double2*)src, S.ldc, (double2*)c->d_stage, S.npw,
                                                     S.d_from_caller, S.d_conj_caller, S.npw, nb);
   AMDK_TRY_HIP(hipGetLastError());
-  AMDK_TRY_HIP(hipMemcpy2DAsync(host, sizeof(double2) * lddst, c->d_stage, sizeof(double2) * S.ldc,
-                                sizeof(double2) * S.npw, nb, hipMemcpyDeviceToHost, c->stream));
-  AMDK_TRY_HIP(hipStreamSynchronize(c->stream));
+  copy_out(c, c->d_stage, host, nb, sizeof(double2) * S.npw, sizeof(double2) * lddst);
 }
 
 // ---------------------------------------------------------------------------
@@ -843,17 +978,11 @@ static void check_nb(amdk_ctx* c, int nb) {
   if (nb < 1 || nb > c->nbmax) throw Error(AMDK_ERR_ARG, "band count outside 1..nbmax");
 }
 
-static void check_finite(const double* p, size_t n, const char* what) {
-  for (size_t i = 0; i < n; ++i)
-    if (!std::isfinite(p[i])) throw Error(AMDK_ERR_NONFINITE, std::string("non-finite value in ") + what);
-}
-
 static void alloc_scf_buffers(amdk_ctx* c);
 static void destroy_scf(amdk_ctx* c);
 static double* noalloc_scratch(int dev);
-static void grid_in(amdk_ctx* c, const double* host, double* dev);
+static void grid_in(amdk_ctx* c, const double* host, double* dev, const char* what);
 static void grid_out(amdk_ctx* c, const double* dev, double* host);
-static void check_finite_grid(const amdk_ctx* c, const double* host, const char* what);
 
 extern "C" {
 
@@ -995,6 +1124,7 @@ int amdk_ctx_create(const amdk_desc* d, amdk_ctx** out) {
     ctx->d_wpair = (double*)dev_alloc(ctx, sizeof(double) * (d->nbmax + 2));
     ctx->d_wdens = (double*)dev_alloc(ctx, sizeof(double) * (d->nbmax + 1));
     alloc_scf_buffers(ctx);
+    copy_setup(ctx, sizeof(double2) * (size_t)S.npw * d->nbmax);
     AMDK_TRY_HIP(hipStreamSynchronize(ctx->stream));
   } catch (const amdk::Error& e) {
     ctx->err = e.what();
@@ -1011,6 +1141,7 @@ void amdk_ctx_destroy(amdk_ctx* ctx) {
   if (!ctx) return;
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   destroy_scf(ctx);
+  copy_destroy(ctx);
   for (void* p : ctx->owned) (void)hipFree(p);
   for (auto& s : ctx->pending) { (void)hipEventDestroy(s.a); (void)hipEventDestroy(s.b); }
   for (hipEvent_t e : ctx->event_pool) (void)hipEventDestroy(e);
@@ -1041,9 +1172,8 @@ int amdk_set_vks(amdk_ctx* ctx, const double* v_r) {
   API_BEGIN
   if (!v_r) throw Error(AMDK_ERR_ARG, "null v_r");
   const size_t nr = (size_t)ctx->n1 * ctx->n2 * ctx->n3;
-  check_finite_grid(ctx, v_r, "v_r");
   double* stage = ctx->grid[1];  // dense scratch grid, free between calls
-  grid_in(ctx, v_r, stage);
+  grid_in(ctx, v_r, stage, "v_r");
   const double s = 1.0 / (double)nr;  // forward FFT normalisation folded into V
   if (ctx->prec == AMDK_PREC_FP64) launch_potential<double>(ctx, stage, s, ctx->yz_vpsi);
   else launch_potential<float>(ctx, stage, s, ctx->yz_vpsi);
@@ -1072,11 +1202,10 @@ int amdk_vpsi(amdk_ctx* ctx, const double* c0, int ldc, double* c2, const double
   if (!c0 || !c2 || !occ) throw Error(AMDK_ERR_ARG, "null pointer");
   if (ldc < ctx->spw.npw) throw Error(AMDK_ERR_ARG, "ldc < ngpw");
   if (!ctx->have_vks) throw Error(AMDK_ERR_STATE, "V_KS not set (amdk_set_vks)");
-  check_finite(c0, (size_t)2 * ldc * nb, "c0");
   // band scratch of the context (C2 and Ct carry no state between calls)
   void* dc0 = ctx->Ct;
   void* dc2 = ctx->C2;
-  bands_in(ctx, c0, ldc, nb, dc0);
+  bands_in(ctx, c0, ldc, nb, dc0, "c0");
   AMDK_TRY_HIP(hipMemcpyAsync(ctx->d_occ, occ, sizeof(double) * nb, hipMemcpyHostToDevice, ctx->stream));
   ctx->occ_state_loaded = false;  // d_occ now holds this call's occupations
   if (ctx->prec == AMDK_PREC_FP64) run_vpsi<double>(ctx, dc0, dc2, nb);
@@ -1103,11 +1232,9 @@ int amdk_density(amdk_ctx* ctx, const double* c0, int ldc, const double* occ, in
   check_nb(ctx, nb);
   if (!c0 || !occ || !rho_r) throw Error(AMDK_ERR_ARG, "null pointer");
   if (ldc < ctx->spw.npw) throw Error(AMDK_ERR_ARG, "ldc < ngpw");
-  check_finite(c0, (size_t)2 * ldc * nb, "c0");
-  const size_t nr = (size_t)ctx->n1 * ctx->n2 * ctx->n3;
   void* dc0 = ctx->Ct;          // band scratch
   double* drho = ctx->grid[0];  // density grid (rewritten before every use)
-  bands_in(ctx, c0, ldc, nb, dc0);
+  bands_in(ctx, c0, ldc, nb, dc0, "c0");
   prepare_density_weights(ctx, occ, nb);
   if (ctx->prec == AMDK_PREC_FP64) run_density<double>(ctx, dc0, nb, drho);
   else run_density<float>(ctx, dc0, nb, drho);

@@ -154,6 +154,7 @@ struct amdk_ctx {
   double* d_wdens = nullptr;  // f_b for the density norm
   double* d_pcg = nullptr;    // PCG scalars
   int* d_info = nullptr;      // directly after d_red[16]
+  int* d_flag = nullptr;      // non-finite input seen (k_check_finite)
   void* h_stage = nullptr;    // pinned host copy of d_red and d_info
   // resident wavefunction state for amdk_scf_step
   void* C0 = nullptr;
@@ -161,7 +162,11 @@ struct amdk_ctx {
   void* Hd = nullptr;
   void* Pd = nullptr;
   void* Ct = nullptr;
-  void* d_stage = nullptr;  // caller-layout staging of host band arrays (ldc x nbmax)
+  void* d_stage = nullptr;  // caller-layout staging of host band arrays (npw x nb, packed)
+  // pinned slots of the threaded copies out (copy_out): two per worker
+  char* h_slots = nullptr;
+  int copy_workers = 0;
+  std::vector<hipEvent_t> copy_ev;
   int nb_state = 0;
   std::vector<double> h_occ_state;
   // d_occ, d_wnorm, d_finv and d_wpair hold the resident state's occupations
