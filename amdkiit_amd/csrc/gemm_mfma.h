@@ -52,7 +52,12 @@ __device__ __forceinline__ void acc_flush(dbl4& hi, flt4& lo) {
   lo = (flt4){0.f, 0.f, 0.f, 0.f};
 }
 
-constexpr int OVM_T = 64, OVM_KT = 64;
+constexpr int OVM_T = 64;
+// K tile of the 64 x 64 form: 64 deep in FP32; 32 in FP64, whose 33 KB of LDS
+// let four blocks share a CU instead of two (S at 64 H2O 0.327 -> 0.300 ms, the
+// FP64 Lagrange overlap at 32 H2O 0.060 -> 0.056; FP32 at 32: fnl at 64 H2O
+// 0.147 -> 0.208).
+template <typename TC> struct OvmTile { static constexpr int KT = sizeof(TC) == 8 ? 32 : 64; };
 
 // MI355X hands consecutive workgroups round-robin to its 8 XCDs, each with
 // its own L2.  Physical block p runs logical block xcd_block(p, per) so that
@@ -62,19 +67,20 @@ constexpr int OVM_T = 64, OVM_KT = 64;
 __device__ __forceinline__ int xcd_block(int p, int per) { return (p & 7) * per + (p >> 3); }
 
 // Block tile 64 x 64 of the result, 4 waves of 32 x 32 (2 x 2 MFMA tiles);
-// logical block = (split, n-tile, m-tile), m fastest.  The next 64-deep K
-// tile is loaded into registers (double2, 512 B per row) while the current
+// logical block = (split, n-tile, m-tile), m fastest.  The next K tile is
+// loaded into registers (double2, 512 B per row) while the current
 // one is multiplied from LDS.  sym (X = Y, M = N) computes only the tiles
 // on and above the diagonal (m-tile <= n-tile, numbered column by column);
 // k_ovl_reduce mirrors them.  A diagonal tile's two operands are the same
 // rows, loaded and staged once.
 template <typename TC>
-__global__ void __launch_bounds__(256) k_ovl_mfma(const double* __restrict__ X, int ldx, int M,
+__global__ void __launch_bounds__(256, sizeof(TC) == 8 ? 4 : 1) k_ovl_mfma(const double* __restrict__ X, int ldx, int M,
                                                   const double* __restrict__ Y, int ldy, int N, int K,
                                                   int kchunk, int nsplit, int per, int sym,
                                                   double* __restrict__ part) {
   typedef typename Acc4<TC>::type AccT;
   constexpr bool F64 = sizeof(TC) == 8;
+  constexpr int OVM_KT = OvmTile<TC>::KT;
   constexpr int KH = OVM_KT / 2;                      // double2 per row and tile
   constexpr int LD = (OVM_T * KH) / 256;              // double2 loads per thread and operand
   __shared__ TC xs[OVM_T][OVM_KT + 1];
@@ -436,9 +442,10 @@ struct UpdNorms {
 // The block's band weights for the norms, staged in LDS before the main
 // loop (so that the epilogue reads no global memory in data-dependent
 // order): wn_s[i] = w_n, fn_s[i] = finv_n for n = n0 + i < nocc, else 0.
+template <int NB>
 __device__ __forceinline__ void upd_norms_stage(const UpdNorms& nm, int n0, double* wn_s, double* fn_s) {
   if (nm.part == nullptr) return;
-  for (int i = threadIdx.x; i < UPM_NB; i += blockDim.x) {
+  for (int i = threadIdx.x; i < NB; i += blockDim.x) {
     const int n = n0 + i;
     const bool ok = n < nm.nocc;
     wn_s[i] = ok ? nm.w[n] : 0.0;
@@ -558,8 +565,10 @@ __global__ void __launch_bounds__(RED_BLOCKS) k_fold_norms_pcg(const double* __r
   if (threadIdx.x == 0) pcg_scalar_set(p2, st, istep);
 }
 
-// Block: 64 reals of k (4 waves x 16) x 128 columns n (8 MFMA tiles per
-// wave); logical block = (k-block, n-block), n fastest, so the n-blocks that
+// Block: 64 reals of k (4 waves x 16) x 16 NT columns n (NT MFMA tiles per
+// wave): NT = 8, or 2 and 4 where all columns fit in 32 and 64, so that a few
+// bands do not pay for 128 (8 bands, 514 plane waves: the Lagrange update 0.015
+// -> 0.010 ms, C U^-1 0.0095 -> 0.0075); logical block = (k-block, n-block), n fastest, so the n-blocks that
 // read the same rows of X share an XCD's L2.  Chunks of 32 m: X (32 x 64)
 // and Q (32 x 128) are staged in LDS, the next chunk prefetched into
 // registers while the current one is multiplied.
@@ -570,7 +579,7 @@ __global__ void __launch_bounds__(RED_BLOCKS) k_fold_norms_pcg(const double* __r
 // (Im c(G = 0) of a Gamma-point band, which must vanish).  TRI declares Q1
 // upper triangular (Q1(m, n) = 0 for m > n): the MFMA tiles whose columns
 // all lie left of a chunk's first row are skipped (their terms are zero).
-template <typename TC, bool TRI>
+template <typename TC, bool TRI, int NT>
 __global__ void __launch_bounds__(256) k_upd_mfma(const double* __restrict__ X1, int ldx, int M1,
                                                   const double* __restrict__ Q1, int ldq1, double a1,
                                                   const double* __restrict__ X2, int M2,
@@ -579,6 +588,7 @@ __global__ void __launch_bounds__(256) k_upd_mfma(const double* __restrict__ X1,
                                                   double beta, int per, int zero_g0_im, UpdNorms nm) {
   typedef typename Acc4<TC>::type AccT;
   constexpr bool F64 = sizeof(TC) == 8;
+  constexpr int UPM_NB = 16 * NT;                  // columns per block
   constexpr int XL = (UPM_MC * UPM_K / 2) / 256;   // double2 of X per thread
   constexpr int QL = (UPM_MC * UPM_NB / 2) / 256;  // double2 of Q per thread
   __shared__ TC qs[UPM_MC][UPM_NB + 1];
@@ -591,11 +601,11 @@ __global__ void __launch_bounds__(256) k_upd_mfma(const double* __restrict__ X1,
   const int li = lane & 15, lk = lane >> 4;
   const int kl = wave * 16 + li, k = k0 + kl;
   __shared__ double wn_s[UPM_NB], fn_s[UPM_NB];
-  upd_norms_stage(nm, n0, wn_s, fn_s);  // visible after the main loop's first barrier
-  dbl4 acc[8];
-  AccT tac[8];
+  upd_norms_stage<UPM_NB>(nm, n0, wn_s, fn_s);  // visible after the main loop's first barrier
+  dbl4 acc[NT];
+  AccT tac[NT];
 #pragma unroll
-  for (int t = 0; t < 8; ++t) {
+  for (int t = 0; t < NT; ++t) {
     acc[t] = (dbl4){0.0, 0.0, 0.0, 0.0};
     tac[t] = (AccT){0, 0, 0, 0};
   }
@@ -642,29 +652,29 @@ __global__ void __launch_bounds__(256) k_upd_mfma(const double* __restrict__ X1,
     if (mb + UPM_MC < M) load(mb + UPM_MC);
     const int mend = min(UPM_MC, M - mb);
     // tiles t < tskip: columns n0 + 16 t + 15 < mb, Q1 = 0 on this chunk
-    const int tskip = (TRI && mb < M1p) ? min(8, max(0, (mb - n0) / 16)) : 0;
+    const int tskip = (TRI && mb < M1p) ? min(NT, max(0, (mb - n0) / 16)) : 0;
     for (int ms = 0; ms < mend; ms += 4) {
       const TC b = xs[ms + lk][kl];
       if constexpr (F64) {
 #pragma unroll
-        for (int t = 0; t < 8; ++t)
+        for (int t = 0; t < NT; ++t)
           if (!TRI || t >= tskip) acc[t] = mfma16(qs[ms + lk][16 * t + li], b, acc[t]);
       } else {
 #pragma unroll
-        for (int t = 0; t < 8; ++t)
+        for (int t = 0; t < NT; ++t)
           if (!TRI || t >= tskip) tac[t] = mfma16(qs[ms + lk][16 * t + li], b, tac[t]);
       }
     }
     if constexpr (!F64) {
 #pragma unroll
-      for (int t = 0; t < 8; ++t) acc_flush(acc[t], tac[t]);
+      for (int t = 0; t < NT; ++t) acc_flush(acc[t], tac[t]);
     }
     __syncthreads();
   }
   if constexpr (TRI) {  // C U^-1 (no norms): the plain store
     if (k < K) {
 #pragma unroll
-      for (int t = 0; t < 8; ++t)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int n = n0 + 16 * t + acc_row<TC>(lk, v);
@@ -675,7 +685,7 @@ __global__ void __launch_bounds__(256) k_upd_mfma(const double* __restrict__ X1,
         }
     }
   } else {
-    upd_store<8>(acc, [](int lk, int v) { return acc_row<TC>(lk, v); }, Y, ldy, N, K, k, n0, lk, beta, zero_g0_im, nm,
+    upd_store<NT>(acc, [](int lk, int v) { return acc_row<TC>(lk, v); }, Y, ldy, N, K, k, n0, lk, beta, zero_g0_im, nm,
                  wn_s, fn_s, L);
   }
 }
@@ -707,7 +717,7 @@ __global__ void __launch_bounds__(256) k_upd_bf16(const double* __restrict__ X1,
   const int li = lane & 15, lk = lane >> 4;
   const int kl = wave * 16 + li, k = k0 + kl;
   __shared__ double wn_s[UPM_NB], fn_s[UPM_NB];
-  upd_norms_stage(nm, n0, wn_s, fn_s);  // visible after the main loop's first barrier
+  upd_norms_stage<UPM_NB>(nm, n0, wn_s, fn_s);  // visible after the main loop's first barrier
   dbl4 acc[8];
   flt4 tac[8];
 #pragma unroll
