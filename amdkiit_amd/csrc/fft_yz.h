@@ -27,6 +27,7 @@
 // place in the plane.  The twiddles W_N^(t j) of a lane stay in registers.
 #pragma once
 #include "fft_reg.h"
+#include "yz_pads.h"
 
 namespace amdk {
 
@@ -38,7 +39,13 @@ template <typename T, int A, int B> struct YzShape {
   static constexpr int CPW = 64 / TM;              // columns per wave
   static constexpr int GZ = (N + CPW - 1) / CPW;   // z groups of a plane
   static constexpr int imin(int a, int b) { return a < b ? a : b; }
-  static constexpr int PS = N + 1, CS = N + 2;     // column strides of the plane and the exchange (odd: no bank pattern)
+  // strides with the fewest bank conflicts: of the plane's columns, of the y
+  // exchange's rows in a column, of the z exchange's columns and rows (against
+  // N + 1 throughout, where half of the LDS cycles were conflicts: k_yz_vpsi and
+  // k_yz_rho at 100^3 FP64 0.346 -> 0.325 and 0.186 -> 0.179 ms, at 144^3 FP32
+  // 0.906 -> 0.826 and 0.689 -> 0.651, at 180^3 4.38 -> 4.02 and 3.91 -> 3.65)
+  using P = YzPads<N, sizeof(V)>;
+  static constexpr int PS = P::PS, RS = P::RS, CS = P::CS, RX = P::RX, RY = P::RY;
   static constexpr size_t plane_values(int nplane) { return (size_t)nplane * PS + 1; }  // and one zero
   static constexpr size_t lds(int nplane, int waves) {
     return (size_t)nplane * sizeof(int4) + plane_values(nplane) * sizeof(V) + (size_t)waves * CPW * CS * sizeof(T);
@@ -89,23 +96,24 @@ __device__ __forceinline__ void wave_lds_sync() {
 
 // Transpose between the two halves of a column transform within the wave:
 // lane t < DA hands in DB values, lane t < DB gets value t of every lane.
-template <int DA, int DB, typename T, typename V>
+// RX: row stride in ex.
+template <int DA, int DB, int RX, typename T, typename V>
 __device__ __forceinline__ void wave_exchange(V* r, T* ex, int t, bool in) {
   const int tr = t < DB ? t : 0;
   wave_lds_sync();
   if (in)
 #pragma unroll
-    for (int j = 0; j < DB; ++j) ex[t * DB + j] = r[j].x;
+    for (int j = 0; j < DB; ++j) ex[t * RX + j] = r[j].x;
   wave_lds_sync();
 #pragma unroll
-  for (int k = 0; k < DA; ++k) r[k].x = ex[k * DB + tr];
+  for (int k = 0; k < DA; ++k) r[k].x = ex[k * RX + tr];
   wave_lds_sync();
   if (in)
 #pragma unroll
-    for (int j = 0; j < DB; ++j) ex[t * DB + j] = r[j].y;
+    for (int j = 0; j < DB; ++j) ex[t * RX + j] = r[j].y;
   wave_lds_sync();
 #pragma unroll
-  for (int k = 0; k < DA; ++k) r[k].y = ex[k * DB + tr];
+  for (int k = 0; k < DA; ++k) r[k].y = ex[k * RX + tr];
 }
 
 // What a block holds besides its pair: LDS and the lane's place in its wave.
@@ -177,11 +185,12 @@ template <typename T, int A, int B, int W> struct YzBlock {
       wave_lds_sync();  // the previous pair's y_forward has read the column
       if (act && t < A)
 #pragma unroll
-        for (int j = 0; j < B; ++j) col[t * B + j] = r[j];
+        for (int j = 0; j < B; ++j) col[t * S::RS + j] = r[j];
       wave_lds_sync();
       const int tr = t < B ? t : 0;
 #pragma unroll
-      for (int k = 0; k < A; ++k) r[k] = col[k * B + tr];
+      for (int k = 0; k < A; ++k) r[k] = col[k * S::RS + tr];
+      wave_lds_sync();  // every lane has read before the column is overwritten
       RDft<V, A, +1>::run(r);
       if (act && t < B)
 #pragma unroll
@@ -203,12 +212,12 @@ template <typename T, int A, int B, int W> struct YzBlock {
       RDft<V, B, -1>::run(r);
       twist<B, -1>(r);
       wave_lds_sync();
-      if (act && t < A)  // value j of lane t where the lane's input t + A j was
+      if (act && t < A)
 #pragma unroll
-        for (int j = 0; j < B; ++j) col[t + A * j] = r[j];
+        for (int j = 0; j < B; ++j) col[t * S::RS + j] = r[j];
       wave_lds_sync();
 #pragma unroll
-      for (int k = 0; k < A; ++k) r[k] = col[k + A * tb];
+      for (int k = 0; k < A; ++k) r[k] = col[k * S::RS + tb];
       RDft<V, A, -1>::run(r);
       const int cnt = act && t < B ? pi.z : 0;
 #pragma unroll
@@ -231,7 +240,7 @@ template <typename T, int A, int B, int W> struct YzBlock {
     }
     RDft<V, B, +1, pencil_zeros<true, A, B>()>::run(r);
     twist<B, +1>(r);
-    wave_exchange<A, B>(r, ex, t, cact && t < A);
+    wave_exchange<A, B, S::RX>(r, ex, t, cact && t < A);
     RDft<V, A, +1>::run(r);
   }
 
@@ -239,7 +248,7 @@ template <typename T, int A, int B, int W> struct YzBlock {
   __device__ __forceinline__ void z_forward(int y, V* r) {
     RDft<V, A, -1>::run(r);
     twist<A, -1>(r);
-    wave_exchange<B, A>(r, ex, t, cact && t < B);
+    wave_exchange<B, A, S::RY>(r, ex, t, cact && t < B);
     RDft<V, B, -1>::run(r);
     const int cnt = cact && t < A && y < N ? np : 0;
 #pragma unroll
