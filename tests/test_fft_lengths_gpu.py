@@ -87,3 +87,27 @@ def test_one_kernel_matches_separate_passes(nb, prec, tol, monkeypatch):
         assert rel(out[key][0], out["passes", None][0]) < tol
         assert rel(out[key][1], out["passes", None][1]) < tol
     assert np.array_equal(out["", None][0], out["", "1"][0])
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("mixed", 2e-6)])
+@pytest.mark.parametrize("n,nb", [(72, 65), (90, 70), (100, 64), (108, 66), (120, 65), (144, 67), (180, 257)])
+def test_many_pairs_in_one_kernel(n, nb, prec, tol, monkeypatch):
+    """The density from the y-z kernel at the lengths and band counts where it
+    is used: pair groups that divide the pairs and that do not, an odd band
+    count, and pairs in several chunks with a short last one (which the chunk
+    before accumulates into)."""
+    pw = sphere_to_the_edge((20, n, n))
+    c = random_bands(pw, nb, seed=7)
+    occ = np.linspace(2.0, 0.5, nb)
+    v = smooth_potential(pw)
+    want = O.eval_density(c, occ, pw.mill_pw, pw.n, pw.cell.omega)
+    want2 = O.vpsi(c, occ, v, pw.mill_pw, pw.n, pw.cell.g)
+    for budget in (None, "40"):
+        if budget:
+            monkeypatch.setenv("AMDK_PAIR_BUDGET_MB", budget)
+        print(f"case=many_pairs n={n} nb={nb} prec={prec} budget={budget}", flush=True)
+        ctx = KSContext(pw, nb, prec)
+        ctx.set_vks(v)
+        assert rel(ctx.eval_density(c, occ), want) < tol
+        assert rel(ctx.vpsi(c, occ), want2) < tol
+        ctx.close()
