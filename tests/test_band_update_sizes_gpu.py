@@ -39,3 +39,25 @@ def test_lagrange_and_ortho(box, ecut, nb, prec, tol):
     assert np.abs(g - ref).max() < tol * np.abs(c2).max() * max(1.0, np.sqrt(nb))
     assert abs(gemax - np.abs(ref).max()) < 10 * tol * np.abs(c2).max()
     ctx.close()
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("mixed", 2e-6)])
+@pytest.mark.parametrize("nb", [5, 18, 50, 66])
+@pytest.mark.parametrize("box,ecut", [(6.0, 8.0), (10.0, 30.0)])
+def test_lagrange_with_empty_bands(box, ecut, nb, prec, tol):
+    """One-launch and split-K overlaps with bands that take no part."""
+    pw = small_setup(box, ecut)
+    if nb > pw.ngpw // 2:
+        pytest.skip("more bands than the sphere can hold")
+    print(f"case=empty_bands nb={nb} npw={pw.ngpw} prec={prec}", flush=True)
+    ctx = KSContext(pw, nb, prec)
+    c = ctx.ortho(random_bands(pw, nb, seed=nb))
+    c2 = random_bands(pw, nb, seed=nb + 500)
+    occ = np.full(nb, 2.0)
+    occ[1::4] = 0.0
+    g, _, _ = ctx.lagrange(c, c2, occ)
+    lam = overlap(c2, c) * np.outer(occ != 0, occ != 0)
+    ref = c2 - lam.T @ c
+    ref[:, 0] = ref[:, 0].real
+    assert np.abs(g - ref).max() < tol * np.abs(c2).max() * max(1.0, np.sqrt(nb))
+    ctx.close()
