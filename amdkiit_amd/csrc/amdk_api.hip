@@ -154,6 +154,9 @@ static void build_sphere(amdk_ctx* c, const int* mill, int ncaller, Sphere& S) {
     k = j;
   }
   S.nrow = (int)S.h_rows.size();
+  S.zero_row_first = S.h_rows[0].m2 == 0 && S.h_rows[0].m3 == 0;
+  S.nrow0 = 0;
+  for (const RowInfo& r : S.h_rows) S.nrow0 += r.m3 == 0;
   // full rows -> slots sorted by (m3, m2)
   struct FR { int m3, m2, row, mirror; };
   std::vector<FR> fr;

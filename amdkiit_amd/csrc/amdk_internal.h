@@ -60,6 +60,8 @@ struct Sphere {
   int* d_conj_caller = nullptr;  // device [ncaller]
   int ncaller = 0;
   bool planes_contiguous = false;  // each plane's rows are consecutive m2
+  bool zero_row_first = false;     // h_rows[0] is (m2, m3) = (0, 0)
+  int nrow0 = 0;                   // half rows with m3 = 0, first in h_rows
 };
 
 }  // namespace amdk

@@ -174,7 +174,7 @@ __global__ void k_vassemble(const int* __restrict__ mill, int ng, int ldc, Recip
   for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < ng; g += gridDim.x * blockDim.x) {
     double gx, gy, gz;
     gvec_of(mill, g, rc, gx, gy, gz);
-    const double2 A1 = p1[g], B1 = p1[ldc + g];
+    const double2 A1 = p1[g], B1 = p2 ? p1[ldc + g] : make_double2(0.0, 0.0);
     double2 v = vg[g];
     v.x += A1.x + gx * B1.y;
     v.y += A1.y - gx * B1.x;

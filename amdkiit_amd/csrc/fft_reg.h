@@ -571,9 +571,18 @@ struct DenseOut {
 
 
 // ---------------------------------------------------------------------------
-// Dense (density-sphere) passes in FP64: two real fields travel as a + i b.
+// Dense (density-sphere) passes in FP64: two real fields travel as a + i b.  A
+// single real field (rho into G space, V_KS out of it) is its own Hermitian
+// half: only the planes m3 = 0 .. R exist (g.nplane = R + 1), the y passes see
+// no others, the x passes transform each row of them once
+// (k_rows_inv_one_r, k_rows_fwd_one_r), and the last z pass takes plane -m3
+// as conj of plane m3.  These launches are bound by latency on small grids and
+// by memory on large ones.  The two transforms into G space of an LDA V_KS
+// 0.054 -> 0.042 ms at 100^3 and 0.091 -> 0.067 at 144^3, the one out of it 0.028
+// -> 0.024 and 0.046 -> 0.038; an SCF step of 32 H2O 0.952 -> 0.938 ms.
 
-// z-FFT exp(-i) of full columns of a(r) + i b(r); keep planes |m3| <= R.
+// z-FFT exp(-i) of full columns of a(r) + i b(r); keep planes |m3| <= R, or
+// 0 .. R of a single field.
 template <int A, int B, int TX>
 __global__ void __launch_bounds__(TX * (A > B ? A : B))
     k_z_fwd_dense_r(PassGeom g, DenseIn in, double2* __restrict__ W2, const double2* __restrict__ twg, int nf,
@@ -594,6 +603,7 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
   W2 += (size_t)f * g.nplane * g.n2 * g.p1;
   for (int i = threadIdx.x; i < N; i += blockDim.x) tw[i] = twg[i];
   __syncthreads();
+  const int kmin = g.nplane == g.R + 1 ? 0 : -g.R;
   double2 r[TM];
 #pragma unroll
   for (int k = 0; k < TM; ++k) r[k] = make_double2(0.0, 0.0);
@@ -609,7 +619,7 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
 #pragma unroll
     for (int j1 = 0; j1 < A; ++j1) {
       const int kz = signed_freq(t + B * j1, N);
-      if (kz >= -g.R && kz <= g.R) W2[((size_t)(kz + g.R) * n2 + y) * g.p1 + x] = r[j1];
+      if (kz >= kmin && kz <= g.R) W2[((size_t)(kz - kmin) * n2 + y) * g.p1 + x] = r[j1];
     }
   }
 }
@@ -637,6 +647,7 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
   W2 += (size_t)f * g.nplane * g.n2 * g.p1;
   for (int i = threadIdx.x; i < N; i += blockDim.x) tw[i] = twg[i];
   __syncthreads();
+  const bool half = g.nplane == g.R + 1;
   double2 r[TM];
 #pragma unroll
   for (int k = 0; k < TM; ++k) r[k] = make_double2(0.0, 0.0);
@@ -644,7 +655,8 @@ __global__ void __launch_bounds__(TX * (A > B ? A : B))
 #pragma unroll
     for (int k2 = 0; k2 < B; ++k2) {
       const int kz = signed_freq(t + A * k2, N);
-      if (kz >= -g.R && kz <= g.R) r[k2] = W2[((size_t)(kz + g.R) * n2 + y) * g.p1 + x];
+      if (kz >= -g.R && kz <= g.R) r[k2] = W2[((size_t)(half ? abs(kz) : kz + g.R) * n2 + y) * g.p1 + x];
+      if (half && kz < 0) r[k2].y = -r[k2].y;
     }
   }
   col_fft<double2, A, B, +1>(r, t, lds, TX, c, tw);
@@ -702,6 +714,81 @@ __global__ void __launch_bounds__(2 * HR * (A > B ? A : B))
       const double2 P = rd[wrap(m1, N)], M = rm[wrap(-m1, N)];
       out[ri.start + e] = make_double2(0.5 * scale * (P.x + M.x), 0.5 * scale * (P.y - M.y));
       out[(size_t)ldc + ri.start + e] = make_double2(0.5 * scale * (P.y + M.y), -0.5 * scale * (P.x - M.x));
+    }
+  }
+}
+
+// x pass inverse of a single real field on the rows with m3 >= 0: transform u
+// is row u, from nrow on the mirror (-m2, 0) of row u - nrow + 1; the rows of
+// m3 = 0 come first, (0, 0) before the others.
+template <int A, int B, int FR>
+__global__ void __launch_bounds__(FR * (A > B ? A : B))
+    k_rows_inv_one_r(PassGeom g, const double2* __restrict__ C, double2* __restrict__ W1, int ntr,
+                     const double2* __restrict__ twg) {
+  constexpr int N = A * B, TM = MaxAB<A, B>::v, ST = N + 1;
+  extern __shared__ unsigned char smem_raw[];
+  double2* tw = reinterpret_cast<double2*>(smem_raw);
+  double2* lds = tw + N;
+  const int t = threadIdx.x % TM, fr = threadIdx.x / TM;
+  const int u = blockIdx.x * FR + fr;
+  const bool live = u < ntr, mirror = u >= g.nrow;
+  for (int i = threadIdx.x; i < N; i += blockDim.x) tw[i] = twg[i];
+  RowInfo ri{};
+  if (live) ri = g.rows[mirror ? u - g.nrow + 1 : u];
+  __syncthreads();
+  double2 r[TM];
+#pragma unroll
+  for (int k = 0; k < TM; ++k) r[k] = make_double2(0.0, 0.0);
+  if (live && t < A) {
+#pragma unroll
+    for (int k2 = 0; k2 < B; ++k2) {
+      const int m1 = signed_freq(t + A * k2, N);
+      const bool conj = mirror || (u == 0 && m1 < 0);  // (0, 0): both halves
+      const int e = (conj ? -m1 : m1) - ri.m1_0;
+      if (e >= 0 && e < ri.cnt) {
+        r[k2] = C[ri.start + e];
+        if (conj) r[k2].y = -r[k2].y;
+      }
+    }
+  }
+  col_fft<double2, A, B, +1>(r, t, lds, 1, fr * ST, tw);
+  if (live && t < B) {
+    double2* out = W1 + (size_t)(mirror ? ri.slot_m : ri.slot_d) * g.p1;
+#pragma unroll
+    for (int j1 = 0; j1 < A; ++j1) out[t + B * j1] = r[j1];
+  }
+}
+
+// x pass forward of a single real field: the direct rows hold all of it.
+template <int A, int B, int FR>
+__global__ void __launch_bounds__(FR * (A > B ? A : B))
+    k_rows_fwd_one_r(PassGeom g, const double2* __restrict__ W1, double2* __restrict__ out, double scale,
+                     const double2* __restrict__ twg) {
+  constexpr int N = A * B, TM = MaxAB<A, B>::v, ST = N + 1;
+  extern __shared__ unsigned char smem_raw[];
+  double2* tw = reinterpret_cast<double2*>(smem_raw);
+  double2* lds = tw + N;
+  const int t = threadIdx.x % TM, fr = threadIdx.x / TM;
+  const int row = blockIdx.x * FR + fr;
+  const bool live = row < g.nrow;
+  for (int i = threadIdx.x; i < N; i += blockDim.x) tw[i] = twg[i];
+  RowInfo ri{};
+  if (live) ri = g.rows[row];
+  __syncthreads();
+  double2 r[TM];
+#pragma unroll
+  for (int k = 0; k < TM; ++k) r[k] = make_double2(0.0, 0.0);
+  if (live && t < A) {
+    const double2* in = W1 + (size_t)ri.slot_d * g.p1;
+#pragma unroll
+    for (int k2 = 0; k2 < B; ++k2) r[k2] = in[t + A * k2];
+  }
+  col_fft<double2, A, B, -1>(r, t, lds, 1, fr * ST, tw);
+  if (live && t < B) {
+#pragma unroll
+    for (int j1 = 0; j1 < A; ++j1) {
+      const int e = signed_freq(t + B * j1, N) - ri.m1_0;
+      if (e >= 0 && e < ri.cnt) out[ri.start + e] = make_double2(scale * r[j1].x, scale * r[j1].y);
     }
   }
 }

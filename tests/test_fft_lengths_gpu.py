@@ -6,9 +6,11 @@ may be left out."""
 import numpy as np
 import pytest
 
+from amdkiit_amd import psp
 from amdkiit_amd.context import KSContext
 from amdkiit_amd.pwgrid import Cell, PWSetup
 from oracle import pw_oracle as O
+from oracle.ks_oracle import KSOracle
 from tests.common import random_bands, smooth_potential
 
 pytestmark = pytest.mark.gpu
@@ -111,3 +113,26 @@ def test_many_pairs_in_one_kernel(n, nb, prec, tol, monkeypatch):
         assert rel(ctx.eval_density(c, occ), want) < tol
         assert rel(ctx.vpsi(c, occ), want2) < tol
         ctx.close()
+
+
+@pytest.mark.parametrize("xc", ["PZ", "PBE"])
+@pytest.mark.parametrize("n", [(20, 24, 30), (54, 64, 80), (90, 48, 100), (36, 108, 50), (120, 32, 72), (144, 40, 60), (160, 20, 96),
+                               (30, 128, 150), (24, 162, 36), (48, 180, 32), (192, 20, 90)], ids=lambda n: "x".join(map(str, n)))
+def test_potential_of_one_field(n, xc):
+    """rho into G space and V_KS out of it as single real fields (the planes
+    m3 >= 0 only), each length on some axis."""
+    pw = sphere_to_the_edge(n)
+    tab = psp.Tables(pw, [psp.gth("Si", "LDA")])
+    tau = np.array([[1.0, 1.5, 2.0]])
+    print(f"case=one_field n={n} ngrho={pw.ngrho} xc={xc}", flush=True)
+    ctx = KSContext(pw, 2, "fp64")
+    ctx.set_species(tab)
+    ctx.set_positions([0], tau)
+    orc = KSOracle(pw, tab, [0], tau, xc, workers=8)
+    u = smooth_potential(pw)
+    rho = 0.05 * np.exp(u / np.abs(u).max())
+    v, e = ctx.vks(rho, xc)
+    want, exc = orc.vks(rho, orc.rhor2g(rho))
+    assert rel(v, want) < 1e-10
+    assert abs(e["exc"] - exc) < 1e-10 * abs(exc)
+    ctx.close()
