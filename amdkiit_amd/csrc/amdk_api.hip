@@ -263,11 +263,13 @@ static void copy_in(amdk_ctx* c, void* dev, const void* host, size_t rows, size_
 // touch of the caller's pages included), so the context's workers take 2 MiB
 // chunks through two pinned slots each, one moved to the caller's array while
 // the DMA fills the other: 64 H2O bands (320 MB) into new memory 31.5 -> 10.7
-// ms, 32 H2O (65 MB) 6.0 -> 2.1 ms.  Below COPY_MIN the plain copy stays:
-// starting the threads takes longer than they save.  The workers live for the
+// ms, 32 H2O (65 MB) 6.0 -> 2.1 ms.  Below COPY_MIN the plain copy stays: there is
+// at most a millisecond to save, and beside the spinning threads of a caller's
+// parallel region the workers lose more (16 MB: fnl and fnonloc of Si64 between
+// two such regions 6.9 ms without them, 8.7-10.3 with).  The workers live for the
 // call; the calling thread is one of them and does all the work if no other
 // can be started.  Returns with the data in the caller's array.
-constexpr size_t COPY_SLOT = 2u << 20, COPY_MIN = 10u << 20;
+constexpr size_t COPY_SLOT = 2u << 20, COPY_MIN = 32u << 20;
 constexpr int COPY_WORKERS = 8;
 
 static void copy_setup(amdk_ctx* c, size_t largest) {

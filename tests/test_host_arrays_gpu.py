@@ -10,8 +10,8 @@ from tests.common import random_bands, smooth_potential
 
 pytestmark = pytest.mark.gpu
 
-# bands of 13,601 plane waves (0.22 MB each): 0.2, 1.3, 10.2 and 14.4 MB
-COUNTS = (1, 6, 47, 66)
+# bands of 13,601 plane waves (0.22 MB each): 0.2, 1.3, 10.2, 14.4, 33.3 and 38.1 MB
+COUNTS = (1, 6, 47, 66, 153, 175)
 
 
 @pytest.fixture(scope="module")
