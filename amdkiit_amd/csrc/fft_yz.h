@@ -9,9 +9,9 @@
 // once.  What bounds it now: in FP32 the vector ALU (k_yz_vpsi at 100^3 issues
 // in 90 % of its cycles), in FP64 LDS (busy 63 % of the time) and the few
 // waves that fit beside a plane.  y and z passes of one SCF step, ms, before
-// and after: 128 bands at 100^3 0.366 -> 0.303 FP32, 0.691 -> 0.534 FP64; 256
-// bands at 144^3 FP32 1.71 -> 1.59; of one H|psi> alone 0.276 -> 0.177, 0.534
-// -> 0.346 and 1.32 -> 0.90.
+// and after: 128 bands at 100^3 0.366 -> 0.292 FP32, 0.691 -> 0.504 FP64; 256
+// bands at 144^3 FP32 1.71 -> 1.48; of one H|psi> alone 0.276 -> 0.171, 0.534
+// -> 0.325 and 1.32 -> 0.826.
 //
 // W1 is transposed for this: [pair][x][slot] with `pitch` slots per x, so that
 // a block reads and writes one contiguous run (the x passes k_rows_inv_t and
