@@ -723,7 +723,7 @@ static YzPlan yz_plan(const amdk_ctx* c, const Sphere& S) {
 }
 
 // Where the y-z kernels are used: a square y-z plane of a register length, a
-// sphere of consecutive rows within a quarter of the grid, LDS room for the
+// sphere of consecutive rows, (0, 0) among them, within a quarter of the grid, LDS room for the
 // plane, and a length at which they measured faster than the separate passes
 // (96 bands, 70 Ry, both forms in turn; passes / y-z kernels).
 // H|psi> by itself gains wherever the transform fills a wave's lanes: 1.43 at
@@ -747,6 +747,10 @@ static bool use_yz_scf(const amdk_ctx* c, int npairs) { return c->yz_scf && npai
 template <typename T>
 static bool yz_fits(const amdk_ctx* c, const Sphere& S) {
   if (c->n2 != c->n3 || !reg_ok(c, c->n1) || !reg_ok(c, c->n2) || !S.planes_contiguous) return false;
+  // YzCols::at counts on the empty place of the (0, 0) row's mirror: without
+  // that row (a list with m3 > 0 throughout also has contiguous planes) the last
+  // slot would be past an x column whose pitch has no room to spare
+  if (!S.zero_row_first) return false;
   if (!quarter_z(S, c->n3) || !quarter_y(S, c->n2)) return false;
   const YzPlan p = yz_plan<T>(c, S);
   return p.lds_v <= LDS_PER_CU && p.lds_r <= LDS_PER_CU;
