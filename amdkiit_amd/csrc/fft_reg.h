@@ -572,14 +572,14 @@ struct DenseOut {
 
 // ---------------------------------------------------------------------------
 // Dense (density-sphere) passes in FP64: two real fields travel as a + i b.  A
-// single real field (rho into G space, V_KS out of it) is its own Hermitian
-// half: only the planes m3 = 0 .. R exist (g.nplane = R + 1), the y passes see
+// single real field (an LDA's rho and v_xc into G space, V_KS out of it) is its
+// own Hermitian half: only the planes m3 = 0 .. R exist (g.nplane = R + 1), the y passes see
 // no others, the x passes transform each row of them once
 // (k_rows_inv_one_r, k_rows_fwd_one_r), and the last z pass takes plane -m3
 // as conj of plane m3.  These launches are bound by latency on small grids and
 // by memory on large ones.  The two transforms into G space of an LDA V_KS
 // 0.054 -> 0.042 ms at 100^3 and 0.091 -> 0.067 at 144^3, the one out of it 0.028
-// -> 0.024 and 0.046 -> 0.038; an SCF step of 32 H2O 0.952 -> 0.938 ms.
+// -> 0.024 and 0.046 -> 0.038.
 
 // z-FFT exp(-i) of full columns of a(r) + i b(r); keep planes |m3| <= R, or
 // 0 .. R of a single field.
