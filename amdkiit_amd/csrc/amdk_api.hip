@@ -2,13 +2,11 @@
 // density drivers behind the C ABI declared in include/amdk.h.
 #include <algorithm>
 #include <array>
-#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <numeric>
-#include <thread>
 #include <tuple>
 
 #include "amdk_ctx.h"
@@ -259,97 +257,11 @@ static void copy_in(amdk_ctx* c, void* dev, const void* host, size_t rows, size_
   AMDK_TRY_HIP(hipMemcpy2DAsync(dev, row_bytes, host, pitch, row_bytes, rows, hipMemcpyHostToDevice, c->stream));
 }
 
-// Out of the device the runtime's copy is one thread's (15-18 GB/s, first
-// touch of the caller's pages included), so the context's workers take 2 MiB
-// chunks through two pinned slots each, one moved to the caller's array while
-// the DMA fills the other: 64 H2O bands (320 MB) into new memory 31.5 -> 10.7
-// ms, 32 H2O (65 MB) 6.0 -> 2.1 ms.  Below COPY_MIN the plain copy stays: there is
-// at most a millisecond to save, and beside the spinning threads of a caller's
-// parallel region the workers lose more (16 MB: fnl and fnonloc of Si64 between
-// two such regions 6.9 ms without them, 8.7-10.3 with).  The workers live for the
-// call; the calling thread is one of them and does all the work if no other
-// can be started.  Returns with the data in the caller's array.
-constexpr size_t COPY_SLOT = 2u << 20, COPY_MIN = 32u << 20;
-constexpr int COPY_WORKERS = 8;
-
-static void copy_setup(amdk_ctx* c, size_t largest) {
-  const int cpus = std::max(1, (int)std::thread::hardware_concurrency());
-  const int n = (int)std::min<size_t>(std::min(COPY_WORKERS, std::max(1, cpus / 2)), largest / (2 * COPY_SLOT));
-  if (n < 2 || largest < COPY_MIN) return;
-  AMDK_TRY_HIP(hipHostMalloc(&c->h_slots, 2 * COPY_SLOT * n, hipHostMallocDefault));
-  c->copy_ev.assign(2 * n, nullptr);
-  for (hipEvent_t& e : c->copy_ev) AMDK_TRY_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  c->copy_workers = n;
-}
-static void copy_destroy(amdk_ctx* c) {
-  for (hipEvent_t e : c->copy_ev)
-    if (e) (void)hipEventDestroy(e);
-  c->copy_ev.clear();
-  if (c->h_slots) (void)hipHostFree(c->h_slots);
-  c->h_slots = nullptr;
-  c->copy_workers = 0;
-}
-
+// Out of the device, by several threads where that pays (host_copy.h).
+// Returns with the data in the caller's array.
 static void copy_out(amdk_ctx* c, const void* dev, void* host, size_t rows, size_t row_bytes, size_t pitch) {
-  const size_t total = rows * row_bytes;
-  if (total < COPY_MIN || c->copy_workers < 2) {
-    AMDK_TRY_HIP(hipMemcpy2DAsync(host, pitch, dev, row_bytes, row_bytes, rows, hipMemcpyDeviceToHost, c->stream));
-    AMDK_TRY_HIP(hipStreamSynchronize(c->stream));
-    return;
-  }
-  if (pitch == row_bytes) {  // one run
-    row_bytes = total;
-    rows = 1;
-  }
-  const size_t per_row = (row_bytes + COPY_SLOT - 1) / COPY_SLOT, nchunk = rows * per_row;
-  std::atomic<size_t> next{0};
-  std::atomic<int> err{(int)hipSuccess};
-  const int nw = (int)std::min<size_t>(c->copy_workers, total / (2 * COPY_SLOT));
-  struct Piece { char* h; const char* d; size_t n; };
-  auto work = [&](int w) noexcept {
-    auto ok = [&](hipError_t e) {
-      if (e != hipSuccess) err = (int)e;
-      return e == hipSuccess;
-    };
-    if (!ok(hipSetDevice(c->device))) return;
-    char* slot[2] = {c->h_slots + 2 * COPY_SLOT * w, c->h_slots + 2 * COPY_SLOT * w + COPY_SLOT};
-    const hipEvent_t ev[2] = {c->copy_ev[2 * w], c->copy_ev[2 * w + 1]};
-    auto fetch = [&](Piece& p, int s) {  // the next chunk into slot s; false: none left, or an error
-      if (err != (int)hipSuccess) return false;
-      const size_t k = next++;
-      if (k >= nchunk) return false;
-      const size_t r = k / per_row, o = (k % per_row) * COPY_SLOT;
-      p = {(char*)host + r * pitch + o, (const char*)dev + r * row_bytes + o, std::min(COPY_SLOT, row_bytes - o)};
-      return ok(hipMemcpyAsync(slot[s], p.d, p.n, hipMemcpyDeviceToHost, c->stream)) && ok(hipEventRecord(ev[s], c->stream));
-    };
-    Piece p[2];
-    bool have = fetch(p[0], 0);
-    for (int i = 0; have; ++i) {
-      const int s = i & 1;
-      have = fetch(p[s ^ 1], s ^ 1);
-      if (!ok(hipEventSynchronize(ev[s]))) return;
-      std::memcpy(p[s].h, slot[s], p[s].n);
-    }
-  };
-  {
-    struct Team {
-      std::vector<std::thread> t;
-      ~Team() {
-        for (auto& x : t) x.join();
-      }
-    } team;
-    try {
-      team.t.reserve(nw - 1);
-      for (int w = 1; w < nw; ++w) team.t.emplace_back(work, w);
-    } catch (const std::exception&) {
-      // fewer workers: the ones that run take all the chunks
-    }
-    work(0);
-  }
-  const hipError_t fin = hipStreamSynchronize(c->stream);  // no slot is in use after the call
-  if (err != (int)hipSuccess)
-    throw Error(AMDK_ERR_DEVICE, std::string("host copy: ") + hipGetErrorString((hipError_t)err.load()));
-  AMDK_TRY_HIP(fin);
+  const hipError_t e = copy_out(c->slots, c->device, c->stream, dev, host, rows, row_bytes, pitch);
+  if (e != hipSuccess) throw Error(AMDK_ERR_DEVICE, std::string("host copy: ") + hipGetErrorString(e));
 }
 
 // *flag = 1 if any of the n values is not finite.  Bound by memory; 2,048
@@ -1133,7 +1045,6 @@ int amdk_ctx_create(const amdk_desc* d, amdk_ctx** out) {
     ctx->d_wpair = (double*)dev_alloc(ctx, sizeof(double) * (d->nbmax + 2));
     ctx->d_wdens = (double*)dev_alloc(ctx, sizeof(double) * (d->nbmax + 1));
     alloc_scf_buffers(ctx);
-    copy_setup(ctx, sizeof(double2) * (size_t)S.npw * d->nbmax);
     AMDK_TRY_HIP(hipStreamSynchronize(ctx->stream));
   } catch (const amdk::Error& e) {
     ctx->err = e.what();
@@ -1150,7 +1061,7 @@ void amdk_ctx_destroy(amdk_ctx* ctx) {
   if (!ctx) return;
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   destroy_scf(ctx);
-  copy_destroy(ctx);
+  ctx->slots.release();
   for (void* p : ctx->owned) (void)hipFree(p);
   for (auto& s : ctx->pending) { (void)hipEventDestroy(s.a); (void)hipEventDestroy(s.b); }
   for (hipEvent_t e : ctx->event_pool) (void)hipEventDestroy(e);

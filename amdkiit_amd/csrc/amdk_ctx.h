@@ -11,6 +11,7 @@
 #include "gemm.h"
 #include "dense.h"
 #include "gemm_mfma.h"
+#include "host_copy.h"
 
 #define AMDK_TRY_HIP(expr)                                                         \
   do {                                                                             \
@@ -163,10 +164,7 @@ struct amdk_ctx {
   void* Pd = nullptr;
   void* Ct = nullptr;
   void* d_stage = nullptr;  // caller-layout staging of host band arrays (npw x nb, packed)
-  // pinned slots of the threaded copies out (copy_out): two per worker
-  char* h_slots = nullptr;
-  int copy_workers = 0;
-  std::vector<hipEvent_t> copy_ev;
+  amdk::CopySlots slots;          // of the threaded copies out
   int nb_state = 0;
   std::vector<double> h_occ_state;
   // d_occ, d_wnorm, d_finv and d_wpair hold the resident state's occupations
