@@ -16,12 +16,21 @@ namespace amdk {
 // touch of the caller's pages included), so workers take 2 MiB chunks through
 // two pinned slots each, one moved to the caller's array while the DMA fills
 // the other: 64 H2O bands (320 MB) into new memory 31.5 -> 10.7 ms, 32 H2O
-// (65 MB) 6.0 -> 2.1 ms.  Below COPY_MIN the plain copy stays: there is at most a
-// millisecond to save, and beside the spinning threads of a caller's parallel
-// region the workers lose more (16 MB: fnl and fnonloc of Si64 between two such
-// regions 6.9 ms without them, 8.7-10.3 with).
-constexpr size_t COPY_SLOT = 2u << 20, COPY_MIN = 32u << 20;
+// (65 MB) 6.0 -> 2.1 ms.
+//
+// Beside the spinning threads of a caller's parallel region a worker may lose its
+// CPU in the middle of a chunk, and the copy waits for it, some milliseconds, whatever
+// its size: the fewer workers, the rarer.  So there are only as many as have COPY_SHARE each, which
+// is two at COPY_MIN, and they sleep for the DMA instead of spinning.  34 MB into
+// touched memory, alone / beside such threads: plain copy 2.3-2.5 / 2.3 ms, eight
+// spinning workers 1.0 / 3.5-4.0, two sleeping ones 1.0 / 1.4-1.9; 66 MB 4.4 / 4.5,
+// 1.8 / 2.7-3.8, five 1.8 / 2.4-3.1.  Only where the threads of two such regions
+// outnumber the CPUs is the plain copy faster, up to 50 MB (34 MB 2.4 against 4.1 ms; eight
+// workers 8.1).  Below COPY_MIN the plain copy stays: there is at most a millisecond to
+// save.
+constexpr size_t COPY_SLOT = 2u << 20, COPY_MIN = 32u << 20, COPY_SHARE = 12u << 20;
 constexpr int COPY_WORKERS = 8;
+static_assert(COPY_MIN / COPY_SHARE >= 2 && COPY_SHARE >= 2 * COPY_SLOT, "work for two, and two slots each");
 
 // Pinned slots (two per worker) of one context, made at the first copy that
 // uses them.  Without them (no pinned memory left, one CPU) the plain copy does
@@ -53,7 +62,7 @@ struct CopySlots {
     if (hipHostMalloc(&p, 2 * COPY_SLOT * n, hipHostMallocDefault) != hipSuccess) return false;
     mem = (char*)p;
     for (hipEvent_t& e : ev)
-      if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+      if (hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventBlockingSync) != hipSuccess) {
         e = nullptr;
         return false;
       }
@@ -88,7 +97,7 @@ inline hipError_t copy_out(CopySlots& slots, int device, hipStream_t stream, con
   const size_t per_row = (row_bytes + COPY_SLOT - 1) / COPY_SLOT, nchunk = rows * per_row;
   std::atomic<size_t> next{0};
   std::atomic<int> err{(int)hipSuccess};
-  const int nw = (int)std::min<size_t>(slots.workers, total / (2 * COPY_SLOT));
+  const int nw = (int)std::min<size_t>(slots.workers, total / COPY_SHARE);  // 2 at least
   struct Piece { char* h; const char* d; size_t n; };
   auto work = [&](int w) noexcept {
     auto ok = [&](hipError_t e) {
