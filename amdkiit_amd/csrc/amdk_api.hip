@@ -602,11 +602,11 @@ static YzCols yz_cols(const Sphere& S) {
 }
 
 // What the y-z kernels need of a context: LDS bytes and resident blocks of
-// H|psi> and of the density, lane-order values and the lane order.
+// H|psi> and of the density, lane-order values, the lengths' rules and the lane order.
 struct YzPlan {
   size_t lds_v = 0, lds_r = 0, native = 0;
   int resident_v = 0, resident_r = 0, zs = 1;
-  double lanes = 0;
+  bool use_vpsi = false, use_scf = false;
   YzOrder order{};
 };
 template <typename T, int A, int B>
@@ -620,7 +620,8 @@ static YzPlan yz_plan_ab(const amdk_ctx* c, const Sphere& S) {
   p.resident_v = 256 * std::max(1, (int)std::min<size_t>(LDS_PER_CU / p.lds_v, 16 / Y::WV));
   p.resident_r = 256 * std::max(1, (int)std::min<size_t>(LDS_PER_CU / p.lds_r, 16 / Y::WR));
   p.zs = Y::ZS;
-  p.lanes = Y::lanes;
+  p.use_vpsi = Y::use_vpsi;
+  p.use_scf = Y::use_scf;
   p.order = YzOrder{c->n1, Y::N, A, B, Y::TM, Y::CPW, Y::GZ};
   return p;
 }
@@ -634,28 +635,15 @@ static YzPlan yz_plan(const amdk_ctx* c, const Sphere& S) {
   }
 }
 
-// Where the y-z kernels are used: a square y-z plane of a register length, a
-// sphere of consecutive rows, (0, 0) among them, within a quarter of the grid, LDS room for the
-// plane, and a length at which they measured faster than the separate passes
-// (96 bands, 70 Ry, both forms in turn; passes / y-z kernels).
-// H|psi> by itself gains wherever the transform fills a wave's lanes: 1.43 at
-// 100^3, 1.33 at 108^3, 1.26 at 144^3 in FP32, 1.60 and 1.38 at 100^3 and 108^3
-// in FP64; with fewer lanes busy (50 = 10 x 5, 60 = 10 x 6, 128 = 16 x 8)
-// 0.84-1.0, but below 40 the two launches saved count for more (1.27 at 32^3),
-// and from 150 on the planes' traffic.
-static bool yz_gains_vpsi(const YzPlan& p, int n) { return n < 40 || n >= 150 || p.lanes >= 0.78; }
-// An SCF step also takes the density from them and saves the separate passes'
-// second use of the planes: 1.04 at 100^3, 1.06 at 90^3 in FP32 and 1.11, 1.07
-// and 1.06 (108^3) in FP64, but 0.92 at 108^3 in FP32 (9 of 12 lanes) and
-// 0.92-0.98 for the smaller grids, whose planes the caches hold.  At 180^3
-// (12 of 15 lanes) 0.98 with 96 bands and 1.04 with 512.
-static bool yz_gains_scf(const YzPlan& p, int n, bool f64) {
-  return f64 ? n >= 90 && p.lanes >= 0.8 : n >= 72 && (p.lanes >= 0.88 || (n >= 180 && p.lanes >= 0.8));
-}
-// With few pairs in flight the density's pair groups do not fill the device
-// (16 pairs at 100^3: 0.111 against 0.103 ms).
-static bool use_yz_scf(const amdk_ctx* c, int npairs) { return c->yz_scf && npairs >= (c->n2 >= 150 ? 128 : 32); }
+// With few pairs in flight the density's pair groups do not fill the device: 16
+// pairs at 100^3 0.111 against 0.103 ms; steps with 32 pairs at 72^3, 80^3 and 90^3 0.97-1.02,
+// 0.98-0.99 and 1.06, with 48 1.02-1.03, 1.02 and 1.10.  Where a block in FP32 has its CU to itself, 32 pairs
+// at 144^3, 160^3 and 180^3 0.99, 1.00 and 1.01, 64 1.02, 1.04 and 1.04.
+static bool use_yz_scf(const amdk_ctx* c, int npairs) { return c->yz_scf && npairs >= c->yz_scf_pairs; }
 
+// Where the y-z kernels can be used: a square y-z plane of a register length, a
+// sphere of consecutive rows, (0, 0) among them, within a quarter of the grid,
+// LDS room for the plane.  YzShape says at which lengths they are.
 template <typename T>
 static bool yz_fits(const amdk_ctx* c, const Sphere& S) {
   if (c->n2 != c->n3 || !reg_ok(c, c->n1) || !reg_ok(c, c->n2) || !S.planes_contiguous) return false;
@@ -665,7 +653,7 @@ static bool yz_fits(const amdk_ctx* c, const Sphere& S) {
   if (!S.zero_row_first) return false;
   if (!quarter_z(S, c->n3) || !quarter_y(S, c->n2)) return false;
   const YzPlan p = yz_plan<T>(c, S);
-  return p.lds_v <= LDS_PER_CU && p.lds_r <= LDS_PER_CU;
+  return p.use_vpsi && p.lds_v <= LDS_PER_CU && p.lds_r <= LDS_PER_CU;
 }
 
 // Pair groups of the density: the count whose blocks fill the device in the
@@ -752,7 +740,7 @@ static void launch_yz_vpsi(amdk_ctx* c, const Sphere& S, int np) {
   const YzPlan p = yz_plan<T>(c, S);
   const int ps = prof_begin(c, "yz_vpsi");
   switch (c->n2) {
-#define AMDK_C(N, A, B) case N: yz_vpsi_ab<T, A, B>(c, S, np, p); break;
+#define AMDK_C(N, A, B) case N: if constexpr (YzShape<T, A, B>::use_vpsi) yz_vpsi_ab<T, A, B>(c, S, np, p); break;
     AMDK_REG_SIZES(AMDK_C)
 #undef AMDK_C
   }
@@ -764,7 +752,7 @@ static void launch_yz_rho(amdk_ctx* c, const Sphere& S, int np, const double* wp
   const YzPlan p = yz_plan<T>(c, S);
   const int ps = prof_begin(c, "yz_rho");
   switch (c->n2) {
-#define AMDK_C(N, A, B) case N: yz_rho_ab<T, A, B>(c, S, np, p, wpair, accumulate); break;
+#define AMDK_C(N, A, B) case N: if constexpr (YzShape<T, A, B>::use_scf) yz_rho_ab<T, A, B>(c, S, np, p, wpair, accumulate); break;
     AMDK_REG_SIZES(AMDK_C)
 #undef AMDK_C
   }
@@ -1005,8 +993,9 @@ int amdk_ctx_create(const amdk_desc* d, amdk_ctx** out) {
     const bool f64 = ctx->prec == AMDK_PREC_FP64;
     const bool fits = ctx->yz_vpsi && (f64 ? yz_fits<double>(ctx, ctx->spw) : yz_fits<float>(ctx, ctx->spw));
     const YzPlan yzp = !fits ? YzPlan{} : f64 ? yz_plan<double>(ctx, ctx->spw) : yz_plan<float>(ctx, ctx->spw);
-    ctx->yz_vpsi = fits && yz_gains_vpsi(yzp, d->n2);
-    ctx->yz_scf = ctx->yz_vpsi && yz_gains_scf(yzp, d->n2, f64);
+    ctx->yz_vpsi = fits;
+    ctx->yz_scf = yzp.use_scf;
+    ctx->yz_scf_pairs = !f64 && yzp.resident_r <= 256 ? 64 : 32;
     const size_t tb = f64 ? sizeof(double) : sizeof(float);
     ctx->vr = dev_alloc(ctx, tb * nr);
     if (ctx->yz_vpsi) ctx->vn = dev_alloc(ctx, tb * yzp.native);

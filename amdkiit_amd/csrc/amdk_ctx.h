@@ -77,6 +77,7 @@ struct amdk_ctx {
   // y and z transforms in one kernel (fft_yz.h; W1 then transposed): for H|psi>
   // by itself, and for the density with what follows it in an SCF step
   bool yz_vpsi = false, yz_scf = false;
+  int yz_scf_pairs = 0;       // band pairs from which a step uses them
   int4* d_planes = nullptr;   // rows of each plane (YzCols::plane)
   double* d_rhopart = nullptr;
   int rho_groups = 1;

@@ -52,9 +52,8 @@ template <typename T, int A, int B> struct YzShape {
   }
   // Waves per block.  Eight where two blocks of the widest sphere share a
   // CU's LDS.  A single block takes all the waves its registers and LDS allow
-  // for H|psi> (16 in FP32, 12 in FP64 or 8), and eight for the density, whose
-  // sums over the rounds of z groups (A doubles a lane and round) then have
-  // 256 registers to live in.  Measured, ms, 8 / 12 / 16 waves: FP32 H|psi>
+  // for H|psi> (16 in FP32, 12 in FP64 or 8), and for the density eight, or 12 from
+  // 150 on.  Measured, ms, 8 / 12 / 16 waves: FP32 H|psi>
   // at 100^3 (128 bands) 0.177 / 0.222 / 0.197, at 144^3 (256 bands) 1.04 /
   // 0.96 / 0.91; FP64 at 100^3 0.382 / 0.350 / 0.587; the density at 100^3
   // FP32 0.127 / 0.131 / 0.140, FP64 0.188 / 0.336 / 0.431, at 144^3 FP32
@@ -65,10 +64,30 @@ template <typename T, int A, int B> struct YzShape {
   // two density blocks share a plane's z groups where one cannot hold the sums
   static constexpr int ZS = (GZ + WR - 1) / WR * A > 60 ? 2 : 1;
   static constexpr int GH = (GZ + ZS - 1) / ZS, NRH = (GH + WR - 1) / WR;
-  // waves per SIMD that the registers are to leave room for
+  // waves per SIMD that the density's registers are to leave room for: 128 of them
+  // a lane where two FP32 blocks are to share the CU, else 256, or 168 with 12 waves
   static constexpr int EUR = two && sizeof(T) == 4 ? 4 : 2;
+  static constexpr int REGS_R = EUR == 4 ? 128 : WR > 8 ? 168 : 256;
+  // share of those that its sums (A doubles a round), a transform and the twiddles take
+  static constexpr double regs = (2.0 * A * NRH + 2.0 * (sizeof(V) / 4) * TM) / REGS_R;
   // share of a wave's lanes that a transform's two halves keep busy
   static constexpr double lanes = CPW * (A + B) / 128.0;
+  // Lengths at which the kernels measured faster than the separate passes (on
+  // spheres of 70 Ry, both forms in turn; passes / y-z kernels).
+  // H|psi> by itself gains wherever the transform fills a wave's lanes: 1.43 at
+  // 100^3, 1.33 at 108^3, 1.26 at 144^3 in FP32, 1.60 and 1.38 at 100^3 and 108^3
+  // in FP64 (96 bands); with fewer lanes busy (50 = 10 x 5, 60 = 10 x 6, 128 = 16 x 8)
+  // 0.84-1.0, but below 40 the two launches saved count for more (1.27 at 32^3),
+  // and from 150 on the planes' traffic.
+  static constexpr bool use_vpsi = N < 40 || N >= 150 || lanes >= 0.78;
+  // An SCF step also takes the density from them and saves the separate passes'
+  // second use of the planes.  It gains where the density's registers hold what
+  // it needs.  FP32, 128 bands: 72^3 1.08, 80^3 1.04, 90^3 1.10, 100^3 1.09, 144^3 1.03,
+  // 160^3 1.04, 180^3 1.04 (0 to 38 registers spilled), but 96^3 0.87, 108^3 0.96,
+  // 120^3 0.94, 150^3 0.90 (62, 70, 113 and 171).  FP64: 90^3 1.15, 100^3 1.14, 108^3 1.11,
+  // 120^3 1.03; 96^3 0.99 with 64 bands and 1.03 with 128 (lanes 0.78).  Smaller grids lose
+  // (FP64 72^3 0.95, 80^3 0.97 with 64 bands): the caches hold their planes.
+  static constexpr bool use_scf = use_vpsi && N >= (sizeof(T) == 8 ? 90 : 72) && lanes >= 0.8 && regs <= 0.8;
   static size_t native(int n1) { return (size_t)n1 * GZ * A * 64; }  // values of one grid in lane order
 };
 

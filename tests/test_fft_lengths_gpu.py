@@ -115,6 +115,28 @@ def test_many_pairs_in_one_kernel(n, nb, prec, tol, monkeypatch):
         ctx.close()
 
 
+@pytest.mark.parametrize("n,nb,edge,precs", [(72, 65, 0.24, ("mixed",)), (80, 65, 0.24, ("mixed",)), (90, 65, 0.24, ("mixed", "fp64")),
+                                             (100, 67, 0.24, ("mixed", "fp64")), (108, 65, 0.24, ("fp64",)),
+                                             (120, 65, 0.24, ("fp64",)), (144, 129, 0.24, ("mixed",)),
+                                             (144, 65, 0.11, ("fp64",)), (160, 129, 0.24, ("mixed",)),
+                                             (180, 131, 0.24, ("mixed",)), (192, 129, 0.205, ("mixed",))])
+def test_density_lengths_of_one_kernel(n, nb, edge, precs):
+    """Every length and precision that takes the density from the y-z kernel,
+    at the band counts from which it does (192^3, and 144^3 in double
+    precision, only on a smaller sphere), and none that does not."""
+    pw = PWSetup(Cell(np.diag([5.0, 0.25 * n, 0.25 * n])), edge * (2 * np.pi / 0.5) ** 2, n=(20, n, n))
+    c = random_bands(pw, nb, seed=9)
+    occ = np.linspace(2.0, 0.5, nb)
+    want = O.eval_density(c, occ, pw.mill_pw, pw.n, pw.cell.omega)
+    for prec, tol in (("fp64", 1e-12), ("mixed", 2e-6)):
+        print(f"case=density_lengths n={n} nb={nb} R={np.abs(pw.mill_pw).max(0)} prec={prec}", flush=True)
+        ctx = KSContext(pw, nb, prec)
+        ctx.profile(True)
+        assert rel(ctx.eval_density(c, occ), want) < tol
+        assert ("yz_rho" in ctx.profile_names()) == (prec in precs)
+        ctx.close()
+
+
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("mixed", 2e-6)])
 @pytest.mark.parametrize("lacks", ["plane m3 = 0", "odd planes"])
 def test_plane_wave_lists_with_empty_planes(lacks, prec, tol):
