@@ -6,7 +6,7 @@ may be left out."""
 import numpy as np
 import pytest
 
-from amdkiit_amd import psp
+from amdkiit_amd import psp, systems
 from amdkiit_amd.context import KSContext
 from amdkiit_amd.pwgrid import Cell, PWSetup
 from oracle import pw_oracle as O
@@ -135,6 +135,66 @@ def test_density_lengths_of_one_kernel(n, nb, edge, precs):
         assert rel(ctx.eval_density(c, occ), want) < tol
         assert ("yz_rho" in ctx.profile_names()) == (prec in precs)
         ctx.close()
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("mixed", 2e-6)])
+def test_several_pairs_per_block(prec, tol, monkeypatch):
+    """67 pairs at 100^3: three (FP32) or six (FP64) to a block of H|psi> and
+    one over, which work on the same planes in LDS in turn, and the density in
+    groups that do not divide them."""
+    pw = sphere_to_the_edge((100, 100, 100))
+    nb = 133
+    c = random_bands(pw, nb, seed=10)
+    occ = np.linspace(2.0, 0.5, nb)
+    v = smooth_potential(pw)
+    out = {}
+    for fft in ("passes", ""):
+        monkeypatch.setenv("AMDK_FFT", fft)
+        print(f"case=several_pairs prec={prec} fft={fft!r}", flush=True)
+        ctx = KSContext(pw, nb, prec)
+        ctx.set_vks(v)
+        ctx.profile(True)
+        out[fft] = (ctx.vpsi(c, occ), ctx.eval_density(c, occ))
+        assert ({"yz_vpsi", "yz_rho"} <= set(ctx.profile_names())) == (fft == "")
+        ctx.close()
+    for got, want in zip(out[""], out["passes"]):
+        assert rel(got, want) < tol
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("mixed", 2e-6)])
+def test_potential_of_a_step_in_a_later_hpsi(prec, tol):
+    """An SCF step by the separate passes leaves V(r) x fastest; an H|psi> by
+    the y-z kernels after it reorders that potential, after one more step the
+    new one, and after a V_KS of its own that."""
+    s = systems.water_box((1, 1, 2), 10.0, 20.0, "PBE")
+    nb = s.nbands
+    other = random_bands(s.pw, nb, seed=11)
+    occ = np.linspace(2.0, 1.0, nb)
+    ctx, ref = KSContext(s.pw, nb, prec), KSContext(s.pw, nb, prec)
+    for x in (ctx, ref):
+        x.set_species(s.tables)
+        x.set_positions(s.sp, s.tau)
+    ctx.wfn_load(ref.ortho(random_bands(s.pw, nb, seed=12)), s.occ)
+    ctx.profile(True)
+
+    def check(what, rho):
+        print(f"case=later_hpsi {what} n={s.pw.n} prec={prec}", flush=True)
+        v, _ = ref.vks(rho, s.xc)
+        assert rel(ctx.vpsi(other, occ), O.vpsi(other, occ, v, s.pw.mill_pw, s.pw.n, s.pw.cell.g)) < tol
+    for it in (1, 2):
+        rho = ref.eval_density(ctx.wfn_store(), s.occ)
+        ctx.scf_step(it, s.xc)
+        check(f"step {it}", rho)
+        check(f"step {it}, again", rho)
+    assert "z_vpsi" in ctx.profile_names() and "yz_vpsi" in ctx.profile_names()
+    rho2 = ref.eval_density(other, occ)
+    ctx.vks(rho2, s.xc)
+    check("V_KS", rho2)
+    rho = ref.eval_density(ctx.wfn_store(), s.occ)
+    ctx.scf_step(3, s.xc)
+    check("step 3", rho)
+    for x in (ctx, ref):
+        x.close()
 
 
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("mixed", 2e-6)])
