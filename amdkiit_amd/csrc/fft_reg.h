@@ -30,7 +30,7 @@ template <> struct Split<18> { static constexpr int P = 2, Q = 9; };
 
 constexpr int gcd_of(int a, int b) { return b == 0 ? a : gcd_of(b, a % b); }
 
-// x exp(DIR 2 pi i m / L) with the eighth turns spelled out
+// x exp(DIR 2 pi i m / L), quarter turns without products
 template <int L, int DIR, typename V>
 __device__ __forceinline__ V mul_root(V a, int m) {
   using T = decltype(a.x);

@@ -6,9 +6,10 @@
 // The separate passes of fft_reg.h move the planes of every band pair through
 // HBM four times per SCF step (for 128 bands at 100^3 in FP64 2.2 of 3.2 GB)
 // and had become bound by that; here a pair's rows are read twice and written
-// once.  What bounds it now: in FP32 the vector ALU (k_yz_vpsi at 100^3 issues
-// in 90 % of its cycles), in FP64 LDS (busy 63 % of the time) and the few
-// waves that fit beside a plane.  y and z passes of one SCF step, ms, before
+// once.  What bounds k_yz_vpsi now, at 100^3: in FP32 the vector ALU (issuing in 90 %
+// of the cycles in which a CU has waves), in FP64 the few waves that fit beside a
+// plane (LDS 56 %, ALU 52 %).  k_yz_rho at 100^3 in FP32 has 128 registers and spills
+// 38, about a third of its HBM traffic.  y and z passes of one SCF step, ms, before
 // and after: 128 bands at 100^3 0.366 -> 0.292 FP32, 0.691 -> 0.504 FP64; 256
 // bands at 144^3 FP32 1.71 -> 1.48; of one H|psi> alone 0.276 -> 0.171, 0.534
 // -> 0.325 and 1.32 -> 0.826.

@@ -68,7 +68,7 @@ __device__ __forceinline__ int xcd_block(int p, int per) { return (p & 7) * per 
 
 // Block tile 64 x 64 of the result, 4 waves of 32 x 32 (2 x 2 MFMA tiles);
 // logical block = (split, n-tile, m-tile), m fastest.  The next K tile is
-// loaded into registers (double2, 512 B per row) while the current
+// loaded into registers (double2; 512 B per row in FP32, 256 in FP64) while the current
 // one is multiplied from LDS.  sym (X = Y, M = N) computes only the tiles
 // on and above the diagonal (m-tile <= n-tile, numbered column by column);
 // k_ovl_reduce mirrors them.  A diagonal tile's two operands are the same
