@@ -105,7 +105,7 @@ inline hipError_t copy_out(CopySlots& slots, int device, hipStream_t stream, con
       if (e != hipSuccess) err.compare_exchange_strong(none, (int)e);
       return e == hipSuccess;
     };
-    if (!ok(hipSetDevice(device))) return;
+    if (w > 0 && !ok(hipSetDevice(device))) return;  // the calling thread keeps its own
     char* slot[2] = {slots.mem + 2 * COPY_SLOT * w, slots.mem + 2 * COPY_SLOT * w + COPY_SLOT};
     const hipEvent_t ev[2] = {slots.ev[2 * w], slots.ev[2 * w + 1]};
     auto fetch = [&](Piece& p, int s) {  // the next chunk into slot s; false: none left, or an error

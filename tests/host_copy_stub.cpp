@@ -8,6 +8,9 @@
 static std::atomic<int> n_alloc{0}, n_event{0}, n_live{0}, n_async{0}, n_plain{0}, n_sync{0};
 static int fail_alloc, fail_event, fail_async;  // the call (from 1) that fails, 0: none
 static std::atomic<int> last{(int)hipSuccess};
+static thread_local int current = 3;  // the thread's device
+static const std::thread::id caller = std::this_thread::get_id();
+static std::atomic<int> n_other{0};   // copies by threads whose device is neither the context's (0) nor the caller's
 
 static hipError_t told(bool fail, hipError_t e) {
   if (fail) last = (int)e;
@@ -38,12 +41,16 @@ hipError_t hipEventDestroy(hipEvent_t e) {
 }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipSetDevice(int d) {
+  current = d;
+  return hipSuccess;
+}
 hipError_t hipStreamSynchronize(hipStream_t) {
   ++n_sync;
   return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+  n_other += current != 0 && std::this_thread::get_id() != caller;
   if (++n_async == fail_async) return told(true, hipErrorInvalidValue);
   std::memcpy(d, s, n);
   return hipSuccess;
@@ -79,6 +86,6 @@ int main(int, char** a) {
   }
   const int workers = slots.workers;
   slots.release();
-  std::printf("%d %d %d %d %d %d %d\n", n_alloc.load(), n_async.load(), n_plain.load(), n_sync.load(), workers,
-              n_live.load(), (int)hipGetLastError());
+  std::printf("%d %d %d %d %d %d %d %d %d\n", n_alloc.load(), n_async.load(), n_plain.load(), n_sync.load(), workers,
+              n_live.load(), (int)hipGetLastError(), current, n_other.load());
 }

@@ -21,7 +21,7 @@ def stub(tmp_path_factory):
         out = subprocess.run([exe] + [str(x) for x in (rows, row_bytes, pitch, calls, alloc, event, copy)], check=True,
                              capture_output=True, text=True, timeout=60).stdout.split("\n")
         return ([tuple(map(int, x.split())) for x in out[:calls]],
-                dict(zip(("allocs", "chunks", "plain", "syncs", "workers", "live", "error"), map(int, out[calls].split()))))
+                dict(zip(("allocs", "chunks", "plain", "syncs", "workers", "live", "error", "device", "other"), map(int, out[calls].split()))))
     return run
 
 
@@ -38,6 +38,13 @@ def test_large_results(stub, rows, row_bytes, pitch):
         assert n["allocs"] == 1 and n["plain"] == 0 and n["chunks"] > 0 and n["syncs"] == 2
     else:
         assert n["plain"] == 2
+
+
+def test_the_callers_device_stays_current(stub):
+    """Workers of their own take the context's device (0); the calling thread,
+    which is on another (3), stays there."""
+    _, n = stub(*SHAPES[2], calls=2)
+    assert n["device"] == 3 and n["other"] == 0
 
 
 def test_small_results_pin_nothing(stub):
